@@ -53,13 +53,14 @@ typedef enum { TI_KV_DENSE = 0, TI_KV_INT8 = 1 } ti_kv_kind;
  *   PREFILL_STAGED    four-wave kernel, K/V tiles staged through registers into LDS
  *   PREFILL_DIRECT    four-wave kernel, direct global -> LDS tile loads (bf16 dense cache,
  *                     head_dim 128, pages of 2^k >= 16 tokens; otherwise staged)
- *   PREFILL_PINGPONG  eight-wave ping-pong kernel (bf16 dense cache, head_dim 128, pages
- *                     of 2^k >= 16 tokens, 256 % (q_heads / kv_heads) == 0)
+ *   PREFILL_PINGPONG  eight-wave ping-pong kernel, 256 packed rows per work-group (bf16 dense
+ *                     cache, head_dim 128, pages of 2^k >= 16 tokens)
  *   PREFILL_PAIRED    four-wave kernel with direct loads whose work-groups each take a
  *                     heavy and a light 32-row q-tile of a causal step (direct-load shapes,
  *                     32 % (q_heads / kv_heads) == 0, the shapes' unsplit two-wave plan)
  *   PREFILL_PAIRED16  the same paired work-groups on sixteen waves of 16 rows each (four
- *                     per SIMD; the default where the paired plan applies) */
+ *                     per SIMD; on a dense cache only launches of up to 256 pairs, where no
+ *                     form of the ping-pong kernel is faster, the default there) */
 typedef enum {
     TI_PATH_AUTO = 0,
     TI_PATH_DECODE = 1,

@@ -1,0 +1,93 @@
+"""The forms of the ping-pong prefill kernel (pa_prefill_pp.hip) that the library picks from the
+launch's 128-row work-groups, W = q-tiles x KV heads x sequences: KSPLIT (two teams of waves
+on every other key tile), SOLO (one team) and SHARED, at the edges of their ranges, dense and
+INT8, head_dim 64 and 128, ragged batches with an empty sequence, heads per KV head that do not
+divide a q-tile. Tolerances against the double-accumulated oracle as everywhere: max abs
+<= 2e-2, for INT8 plus one bf16 unit of the reference value."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import tileinfer_hip as ti
+from helpers import randn, rng, smoothing
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+BE = ti.HipBackend()
+
+# name: (cache, D, heads, kv_heads, page_size, sequences (start, n), causal)
+CASES = {
+    "paired16_ragged": ("bf16", 128, 32, 8, 16, [(700, 40), (0, 130), (0, 0)], True),   # W = 120: none
+    "ksplit_dense_first": ("bf16", 128, 32, 8, 16, [(0, 520)], True),            # W = 136
+    "ksplit_dense_odd_tiles": ("bf16", 128, 32, 8, 64, [(33, 700)], True),
+    "ksplit_dense_non_causal": ("bf16", 128, 32, 8, 16, [(77, 641)], False),
+    "ksplit_dense_g3": ("bf16", 128, 24, 8, 32, [(10, 850)], True),              # 42 positions a q-tile
+    "ksplit_dense_ragged": ("bf16", 128, 32, 8, 16, [(700, 40), (0, 130), (0, 0), (900, 1), (5, 300)], True),
+    "ksplit_dense_two_tiles": ("bf16", 128, 32, 8, 16, [(60 * (b % 4), 33 + b) for b in range(16)], True),
+    "ksplit_dense_d64": ("bf16", 64, 32, 8, 32, [(5, 700)], True),
+    "ksplit_dense_d64_non_causal": ("bf16", 64, 16, 8, 16, [(100, 650), (0, 650)], False),
+    "ksplit_int8_first": ("int8", 128, 32, 8, 16, [(0, 1030)], True),            # W = 264
+    "ksplit_int8_ragged": ("int8", 128, 32, 8, 64, [(300, 299), (0, 31), (0, 0), (65, 300), (1, 1)], True),
+    "ksplit_int8_d64": ("int8", 64, 16, 8, 16, [(33, 640), (0, 600)], True),
+    "solo_dense_short": ("bf16", 128, 32, 8, 16, [(17 * b, 129 + b) for b in range(16)], True),
+    "solo_dense_two_tiles": ("bf16", 128, 32, 8, 16, [(3 * b, 33 + b % 8) for b in range(32)], True),
+    "solo_dense_d64": ("bf16", 64, 32, 8, 64, [(0, 700), (100, 300), (0, 0), (900, 650)], True),
+    "solo_dense_d64_non_causal": ("bf16", 64, 32, 8, 16, [(31, 500), (0, 320), (7, 513), (64, 33), (0, 1)], False),
+    "solo_int8": ("int8", 128, 32, 8, 16, [(0, 700), (333, 650), (0, 0), (12, 32)], True),
+    "solo_int8_d64": ("int8", 64, 32, 8, 32, [(0, 700), (333, 650), (1, 1), (12, 32)], True),
+    "shared_dense": ("bf16", 128, 32, 8, 16, [(5, 600), (0, 601), (950, 2), (0, 0)], True),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_prefill_form(gpu, name):
+    """Also with NaN in every pool row (INT8: scale) that no sequence holds, which tiles past a
+    step's last key read: none may reach the output."""
+    kind, D, H, KVH, P, seqs, causal = CASES[name]
+    g = rng(5200 + list(CASES).index(name))
+    used = [-(-(s + n) // P) for s, n in seqs]
+    pages, nmax = sum(used) + 3, max(n for _, n in seqs)
+    perm = (g.permutation(pages) + 1).astype(np.int32)
+    bts = np.zeros((len(seqs), max(used) + 2), np.int32)
+    rows = np.zeros((pages, P), bool)               # rows that hold a key
+    at = 0
+    for b, (s, n) in enumerate(seqs):
+        bts[b, :used[b]] = perm[at:at + used[b]]
+        at += used[b]
+        for p in range(s + n):
+            rows[bts[b, p // P] - 1, p % P] = True
+    counts = [n for _, n in seqs]
+    qsl = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    positions = np.concatenate([np.arange(s, s + n) for s, n in seqs]).astype(np.int32)
+    q = randn(g, sum(counts), H, D, bf16=True)
+    kp, vp = randn(g, pages, KVH, P, D, bf16=True), randn(g, pages, KVH, P, D, bf16=True)
+    qd, scale = torch.from_numpy(q).bfloat16().cuda(), 1 / math.sqrt(D)
+    stale = torch.from_numpy(~rows).cuda()[:, None].expand(pages, KVH, P)
+    if kind == "int8":
+        cs = smoothing(g, D)
+        k, v = ti.int8_kv_pools(D, P, KVH, pages, key_smoothing=torch.from_numpy(cs))
+        flat = [torch.from_numpy(np.ascontiguousarray(x.transpose(0, 2, 1, 3).reshape(-1, KVH, D))).bfloat16().cuda()
+                for x in (orc.bf16_round(kp * orc.bf16_round(cs)), vp)]
+        ti.store_kv_(BE, k, v, *flat, torch.arange(1, P * pages + 1, dtype=torch.int32, device="cuda"))
+        pools = dict(layer_q=k.layer_q.cpu().numpy(), layer_scale=k.layer_scale.cpu().numpy(), smooth=cs)
+        for half in range(2):
+            k.layer_scale[half][stale] = float("nan")
+    else:
+        k, v = torch.from_numpy(kp).bfloat16().cuda(), torch.from_numpy(vp).bfloat16().cuda()
+        pools = dict(k_pages=kp, v_pages=vp)
+        k[stale] = float("nan")
+        v[stale] = float("nan")
+    out = torch.full_like(qd, float("nan"))
+    print(f"case {name}", flush=True)
+    ws = ti.attention_workspace(BE, qd, k, num_seqs=len(seqs), max_query_len=nmax)
+    ti.paged_attention_(BE, out, ws, qd, k, v, torch.from_numpy(bts).cuda(), torch.from_numpy(positions).cuda(), scale,
+                        causal, query_start_loc=torch.from_numpy(qsl).cuda() if len(seqs) > 1 else None, max_query_len=nmax)
+    got = out.float().cpu().numpy()
+    for b, (s, n) in enumerate(seqs):
+        if n == 0:
+            continue
+        ref = orc.attention(q[qsl[b]:qsl[b + 1]], bts[b], s, scale, causal, **pools)
+        excess = np.abs(ref - got[qsl[b]:qsl[b + 1]]) - (2e-2 + (np.abs(ref) * 2.0 ** -8 if kind == "int8" else 0))
+        assert float(np.max(excess)) <= 0, f"sequence {b}: over the tolerance by {np.max(excess)}"

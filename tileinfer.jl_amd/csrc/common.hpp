@@ -148,8 +148,11 @@ int ti_launch_decode(const ti_attention_args *a, const ti_kv_cache *c, const ti_
 int ti_launch_combine(const ti_attention_args *a, const ti_kv_cache *c, int rows, int splits,
                       hipStream_t s, int flat = 0, int *meta = nullptr, int min_tiles = 0);
 
+// Forms of the ping-pong prefill kernel: two teams of four waves on 256 rows (SHARED) or on
+// the same 128 rows and every other key tile (KSPLIT), or one team on 128 rows (SOLO).
+enum { TI_PP_NONE = 0, TI_PP_SHARED = 1, TI_PP_KSPLIT = 2, TI_PP_SOLO = 3 };
 struct ti_prefill_plan {
-    int pp;          // 1: the 8-wave ping-pong kernel (pa_prefill_pp.hip)
+    int pp;          // a form of the ping-pong kernel (pa_prefill_pp.hip), or TI_PP_NONE
     int dl;          // 1: direct global -> LDS tile loads in the four-wave kernel
     int pair;        // 1: paired heavy / light 32-row q-tiles per work-group (TQ, qtiles per 32 rows)
     int r16;         // 1 (with pair): the paired work-groups on 16-row waves (prefill16_kernel)
@@ -166,7 +169,8 @@ struct ti_prefill_plan {
 ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c, bool bound_keys);
 int ti_launch_prefill(const ti_attention_args *a, const ti_kv_cache *c, const ti_prefill_plan &p,
                       hipStream_t s);
-bool ti_prefill_pp_eligible(const ti_attention_args *a, const ti_kv_cache *c);
+// The ping-pong form a prefill on `path` takes (AUTO, PREFILL: the library's pick).
+int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path);
 int ti_launch_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, const ti_prefill_plan &p,
                          hipStream_t s);
 // fp32 path: its key splits and workspace bytes (host shapes only).

@@ -1213,16 +1213,13 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     const int G = a->q_heads / c->kv_heads;
     const long long pairs = (long long)c->kv_heads * a->num_seqs;
     const long long key_tiles = ((long long)a->block_table_stride * c->page_size + 31) / 32;
-    // The 8-wave ping-pong kernel (256 packed rows per work-group, one per CU) is taken
-    // when its work-groups fill the 256 CUs at least twice without key splits: measured
-    // 906 vs 745 TFLOP/s at a 4096-token causal prefill (512 work-groups), but slower
-    // at 2048 tokens (256) and below, where the four-wave kernel's smaller q-tiles and
-    // in-work-group key groups keep more CUs busy. TI_PATH_PREFILL_PINGPONG pins it
-    // wherever the shapes allow; the other pinned variants never take it.
-    const long long pp_wgs = (long long)((a->max_query_len + 256 / G - 1) / (256 / G)) * pairs;
-    const bool pp_ok = ti_prefill_pp_eligible(a, c);
-    pl.pp = pp_ok && (a->path == TI_PATH_PREFILL_PINGPONG ||
-                      ((a->path == TI_PATH_PREFILL || a->path == TI_PATH_AUTO) && pp_wgs >= 512));
+    // PAIRED16 pins the 16-row kernel where it is not beaten: launches that the library gives
+    // to the ping-pong kernel on a dense cache fall back to that pick.
+    int path = a->path;
+    if (path == TI_PATH_PREFILL_PAIRED16 && c->kind == TI_KV_DENSE && ti_pick_prefill_pp(a, c, TI_PATH_AUTO))
+        path = TI_PATH_AUTO;
+    const bool auto_path = path == TI_PATH_PREFILL || path == TI_PATH_AUTO;
+    pl.pp = ti_pick_prefill_pp(a, c, path);
     pl.dl = 0;
     pl.pair = 0;
     pl.r16 = 0;
@@ -1232,11 +1229,11 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
         // block tables can hold.
         pl.wpg = 8;
         pl.ng = 1;
-        pl.TQ = 256 / G;
+        pl.TQ = (pl.pp == TI_PP_SHARED ? 256 : 128) / G;
         pl.qtiles = (a->max_query_len + pl.TQ - 1) / pl.TQ;
         const long long wgs = (long long)pl.qtiles * pairs;
         pl.splits = 1;
-        while (pl.splits < 16 && wgs * pl.splits < 256 && (!bound_keys || key_tiles / (2 * pl.splits) >= 8))
+        while (!auto_path && pl.splits < 16 && wgs * pl.splits < 256 && (!bound_keys || key_tiles / (2 * pl.splits) >= 8))
             pl.splits *= 2;
         pl.rows = G * a->max_query_len;
         pl.bytes = pl.splits == 1 ? 0 : (size_t)pairs * pl.splits * pl.rows * (c->head_dim + 2) * sizeof(float);
@@ -1261,9 +1258,9 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     // (1024-3072 tokens) no change, so those keep the register-staged loads.
     const bool dl_ok = c->kind == TI_KV_DENSE && a->dtype == TI_BF16 && c->head_dim == 128 &&
                        c->page_size >= 16 && (c->page_size & (c->page_size - 1)) == 0;
-    pl.dl = dl_ok && (a->path == TI_PATH_PREFILL_DIRECT || a->path == TI_PATH_PREFILL_PAIRED ||
-                      a->path == TI_PATH_PREFILL_PAIRED16 ||
-                      (a->path != TI_PATH_PREFILL_STAGED && pl.wpg == 2));
+    pl.dl = dl_ok && (path == TI_PATH_PREFILL_DIRECT || path == TI_PATH_PREFILL_PAIRED ||
+                      path == TI_PATH_PREFILL_PAIRED16 ||
+                      (path != TI_PATH_PREFILL_STAGED && pl.wpg == 2));
     // Paired q-tiles (a heavy and a light 32-row q-tile per work-group, equal causal work
     // per work-group) for causal steps without key splits on the direct-load shapes; G
     // must divide 32 (whole positions per 32-row q-tile). On 16-row waves
@@ -1271,7 +1268,8 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     // plan's four-wave kernel (same process) 11.4 -> 10.4 us at 512 tokens, 22.0 -> 19.7 us
     // for 512 on a 1024-token prefix, 27.2 -> 24.6 us at 1024 tokens, 46.3 -> 42.9 us for
     // 1024 on 1024, even at 768 tokens (384 work-groups), but 37.0 -> 43.3 us at 1536 tokens
-    // (768) and twice as slow from 2048 tokens. The 32-row paired kernel (pinned with
+    // (768) and twice as slow from 2048 tokens. On a dense cache the ping-pong kernel takes
+    // launches of more than 256 pairs first. The 32-row paired kernel (pinned with
     // TI_PATH_PREFILL_PAIRED) needs the plan's two-wave, four-group shape.
     // (INT8 caches pair on the 16-row kernel only, its tiles staged through registers)
     const bool i8_ok = c->kind == TI_KV_INT8 && a->dtype == TI_BF16 && c->head_dim == 128 &&
@@ -1279,10 +1277,9 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     const bool pair_ok = (dl_ok || i8_ok) && a->causal && pl.splits == 1 && 32 % G == 0;
     // (32 % G == 0 in pair_ok: G <= 32, so 32 / G >= 1)
     const long long pair_wgs = pair_ok ? pairs * (((a->max_query_len + 32 / G - 1) / (32 / G) + 1) / 2) : 0;
-    const bool auto_path = a->path == TI_PATH_PREFILL || a->path == TI_PATH_AUTO;
-    pl.r16 = pair_ok && (a->path == TI_PATH_PREFILL_PAIRED16 || (auto_path && R16_BY_DEFAULT && pair_wgs <= 512));
+    pl.r16 = pair_ok && (path == TI_PATH_PREFILL_PAIRED16 || (auto_path && R16_BY_DEFAULT && pair_wgs <= 512));
     pl.pair = pl.r16 || (pair_ok && dl_ok && pl.dl && pl.wpg == 2 && pl.ng == 4 &&
-                         (a->path == TI_PATH_PREFILL_PAIRED || (auto_path && PAIR_BY_DEFAULT)));
+                         (path == TI_PATH_PREFILL_PAIRED || (auto_path && PAIR_BY_DEFAULT)));
     if (pl.pair) {
         pl.TQ = 32 / G;
         pl.qtiles = (a->max_query_len + pl.TQ - 1) / pl.TQ;

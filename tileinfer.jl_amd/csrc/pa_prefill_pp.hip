@@ -1,35 +1,43 @@
 // Paged causal / chunked / non-causal prefill attention, ping-pong form (gfx950, bf16
-// MFMA, dense bf16 cache, head_dim 128, power-of-two pages of >= 16 tokens).
+// MFMA, dense bf16 or INT8 cache, head_dim 64 or 128, power-of-two pages of >= 16 tokens).
 //
-// Reference: attention_prefill_kernel / prefill_body (src/ops/tile/attention.jl:130-177).
-// Query t of the step sits at position start + t (start = positions of the sequence's
-// first query, read on the device) and sees keys 0 .. start + t; with causal = 0 it sees
-// all start + n keys (attention.jl:155-157).
+// Reference: attention_prefill_kernel / prefill_body (src/ops/tile/attention.jl:130-177)
+// and attention_prefill_int8_kernel (:139-147). Query t of the step sits at position
+// start + t (start = positions of the sequence's first query, read on the device) and sees
+// keys 0 .. start + t; with causal = 0 it sees all start + n keys (attention.jl:155-157).
 //
-// Why a second prefill kernel. Per 32-key step a wave holding 32 packed query rows
-// issues 16 v_mfma_f32_32x32x16_bf16 (about 512 matrix-core cycles) and about 100 VALU
-// instructions of softmax (16 of them v_exp_f32; about 500 issue cycles). When every wave
-// of a SIMD enters each phase together the two costs add up. Here a work-group is 8 waves
-// in two teams of 4 (team A = waves 0-3, team B = waves 4-7; wave w runs on SIMD w % 4,
-// so each SIMD holds one wave of each team). Work-group barriers split time into
-// phases; in every phase one team runs its MFMAs (QK^T of tile i and PV of tile i-1) while
-// the other runs the softmax of its last score tile, so each SIMD's matrix core and VALU
-// work at the same time. Team B runs one phase behind team A:
+// A work-group is one or two teams of 4 waves (team A = waves 0-3, team B = waves 4-7; wave w
+// runs on SIMD w % 4, so each SIMD holds one wave of each team). Every wave owns 32 packed
+// query rows. With two teams, work-group barriers split time into phases; in every phase one team runs its
+// MFMAs while the other runs its softmax, so each SIMD's matrix core and VALU work at the
+// same time. Team B runs one phase behind team A:
 //
 //   phase      0      1      2      3      4     ...
 //   team A    X0     Y0     X1     Y1     X2
 //   team B    --     X0     Y0     X1     Y1
 //
-//   X_i = S_i = K_i Q^T (8 MFMAs) and O += V_{i-1} P_{i-1} (8 MFMAs)
-//   Y_i = online softmax of S_i -> P_i (bf16), lazy rescale of O; K/V staging duties
+//   X_i = S_i = K_i Q^T and O += V_{i-1} P_{i-1}, and in the MFMAs' shadow everything else
+//         that is not softmax: V operands of tile i - 1 and K operands of tile i + 1 from
+//         LDS, staged tiles into LDS, global loads of later tiles
+//   Y_i = online softmax of S_i -> P_i (bf16), lazy rescale of O
 //
-// All 8 waves share every 32-key K/V tile in LDS (256 packed query rows per tile, twice
-// the reuse of a 4-wave group). Each thread moves one 16-byte chunk of K and one of V per
-// tile: global loads are issued three steps before the tile's V part is needed, K goes to
-// LDS two steps ahead, V one step ahead; K and V each live in a three-tile LDS ring (a
-// buffer is rewritten only after both teams have read it). Team A's threads carry keys
-// 0-15 of a tile and team B's keys 16-31, so a tile's halves are stored in consecutive
-// phases and each wave's block-table lookup is a single scalar load.
+// Three forms (ti_pick_prefill_pp below has the rule and the figures):
+//   SHARED  all 8 waves share each 32-key tile (256 packed rows per work-group);
+//   KSPLIT  both teams hold the same 128 rows and take every other tile each (team t: tiles
+//           t, t + 2, ...), merged through LDS at the end: half the rows per work-group and
+//           half the steps, for launches whose 256-row tiles leave CUs idle;
+//   SOLO    one team on 128 rows, one barrier a step; two work-groups (head_dim 64: three)
+//           share a CU and overlap each other's phases, first loads and stores.
+//
+// What bounds it. On a full chip, power: a loop of these MFMAs alone runs at 1.5-1.7 GHz (0.70
+// us a SHARED step, 8 waves x 16 MFMAs of 32 cycles, against 0.45 us on 8 CUs at 2.4 GHz), and
+// every instruction saved shows. A SHARED step takes 0.95 us at 8192 tokens (LDS reads of all
+// operands 128 KB a step at 256 B per cycle and CU: not the limit). The MFMA phase used to wait
+// for its operands: keys read in pairs just before their MFMAs, softmax phases carrying the
+// staging. With the keys' operands read a phase ahead, the values' behind the first scores,
+// score and value MFMAs taking turns and everything else in the gaps between them: 8192 tokens
+// 539 -> 493 us (1115 TFLOP/s; bf16 GEMMs of this size reach 1350-1600 here), 4096 tokens
+// 146 -> 135, 2000 on 4000 204 -> 165 (same process, graph replays, inputs of unit variance).
 //
 // The per-wave MFMA layouts, the exp2-domain online softmax with lazy rescale, the
 // transposing V reads and the output / split-partial formats are those of the
@@ -44,13 +52,7 @@ using namespace ti;
 
 namespace {
 
-constexpr int D = 128;
 constexpr int KT = 32;                 // keys per tile
-constexpr int NW = 8;                  // waves per work-group
-constexpr int ROWS = 32 * NW;          // packed query rows per work-group
-constexpr int NBUF = 3;                // LDS ring depth (K and V each)
-constexpr int KROW = D + 8;            // K row stride (bf16): 16-B reads by 16 keys hit 64 banks
-constexpr int VROW = D + 32;           // V row stride: transposing reads bank-disjoint
 constexpr float RESCALE_LOG2 = 8.0f;   // lazy-rescale threshold
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -60,15 +62,24 @@ struct PPParams {
     const uint16_t *q;
     uint16_t *out;
     const uint16_t *kp, *vp;
+    const int8_t *lq;
+    const float *ls, *smooth;
     const int32_t *positions, *qsl, *bt;
     float *part;                       // split partials [B][Hk][splits][M][D + 2]
-    int bt_stride, num_pages, P, pshift, Hk, Hq, G, TQ, nmax, qtiles, causal, splits, M;
+    int bt_stride, num_pages, P, pshift, Hk, Hq, G, TQ, nmax, qtiles, causal, splits, sshift, M;   // splits = 2^sshift
     float scale_log2;
 };
 
-struct PPSmem {
-    uint16_t k[NBUF][KT * KROW];
-    uint16_t v[NBUF][KT * VROW];
+// One tile stream's double-buffered tiles. Row strides (bf16): D + 8 for K (16-B reads by 16
+// keys hit 64 banks), D + 32 for V (transposing reads bank-disjoint). INT8: each tile's key
+// scales (times scale_log2) and value scales, in a four-tile ring (staged with the keys, two
+// tiles ahead, and read by the softmax).
+template <int D, bool INT8>
+struct PPTiles {
+    static constexpr int KROW = D + 8, VROW = D + 32;
+    uint16_t k[2][KT * KROW];
+    uint16_t v[2][KT * VROW];
+    float s[INT8 ? 4 : 1][INT8 ? 2 * KT : 4];
 };
 
 __device__ __forceinline__ u32x2 lds_tr16(const uint16_t *p) {
@@ -79,36 +90,94 @@ __device__ __forceinline__ u32x2 lds_tr16(const uint16_t *p) {
 
 template <int I> using IC = std::integral_constant<int, I>;
 
-__global__ void __launch_bounds__(64 * NW) prefill_pp_kernel(PPParams p) {
+// f(IC<0>{}), ..., f(IC<N - 1>{})
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void unroll(F &&f) {
+    if constexpr (I < N) {
+        f(IC<I>{});
+        unroll<N, I + 1>(f);
+    }
+}
+
+template <int D, bool INT8, int FORM>
+__global__ void __launch_bounds__(FORM == TI_PP_SOLO ? 256 : 512, FORM == TI_PP_SOLO && D == 64 ? 3 : 2)
+prefill_pp_kernel(PPParams p) {
+    constexpr bool KS = FORM == TI_PP_KSPLIT, SOLO = FORM == TI_PP_SOLO;
+    static_assert(D == 128 || KS || SOLO, "head_dim 64 stages a tile with one team");
+    constexpr int NW = SOLO ? 4 : 8;
     constexpr int NQB = D / 16;        // score MFMAs per tile (16 head-dim elements each)
     constexpr int NDB = D / 32;        // 32-row blocks of O^T
-    __shared__ __attribute__((aligned(16))) PPSmem sm;
+    constexpr int RW = KS || SOLO ? 128 : 256; // packed query rows per work-group
+    constexpr int GT = KS || SOLO ? 256 : 512; // threads that stage a tile
+    constexpr int CPR = D / 8;         // 8-element chunks per row
+    constexpr int NC = KT * CPR / GT;  // chunks of K and of V per thread and tile
+    // Steps between a value chunk's load and its store into LDS (keys: 2). The 128-row form at
+    // D = 128 stages two chunks per thread and has registers for one step's values only.
+    constexpr int LV = D == 128 && GT == 256 ? 1 : 2;
+    using Tiles = PPTiles<D, INT8>;
+    using Chunk = std::conditional_t<INT8, u32x2, u32x4>;
+    constexpr int KROW = Tiles::KROW, VROW = Tiles::VROW;
+    constexpr int SLAB = KS ? NW * 64 * (NDB / 2 * 64 + 8) : 0;   // the merge's exchange area (bytes)
+    constexpr int TILES = (KS ? 2 : 1) * (int)sizeof(Tiles);
+    __shared__ __attribute__((aligned(16))) char smem_raw[TILES > SLAB ? TILES : SLAB];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int team = w >> 2;                       // 0: A, 1: B
+    const int team = SOLO ? 0 : w >> 2;                       // 0: A, 1: B
     const int r32 = lane & 31, kg = lane >> 5;
-    const int h = blockIdx.x;
-    const int qt = p.qtiles - 1 - (int)blockIdx.y / p.splits;   // heaviest q-tiles first
-    const int split = (int)blockIdx.y % p.splits;
-    const int b = blockIdx.z;
+    Tiles &sm = reinterpret_cast<Tiles *>(smem_raw)[KS ? team : 0];
+    // Grid (Hk, q-tiles x splits, B): consecutive work-groups (dealt round-robin to the 8 XCDs)
+    // belong to different KV heads, so each head's K/V stays in one XCD's L2.
+    const int h = blockIdx.x, b = blockIdx.z;
+    const int qt = p.qtiles - 1 - (int)(blockIdx.y >> p.sshift);   // heaviest q-tiles first
+    const int split = (int)blockIdx.y & (p.splits - 1);
+    // the pointer arguments the prologue dereferences, in the kernel arguments' first batch
+    asm volatile("" ::"s"(p.bt), "s"(p.positions), "s"(p.qsl), "s"(p.kp), "s"(p.vp), "s"(p.q));
+    const int32_t *bt = p.bt + (size_t)b * p.bt_stride;
+    // This thread's staging chunks: key ckey + (GT / CPR) u, elements cch * 8 .. + 8. A wave's
+    // chunk u lies in one 16-key half of the tile (half_of), so its row base is scalar.
+    const int gt = tid % GT, ckey = gt / CPR, cch = gt % CPR;
+    constexpr int KPU = GT / CPR;
+    const int wave_half = __builtin_amdgcn_readfirstlane(ckey >> 4);
+    auto half_of = [&](int u) { return NC == 2 ? u : wave_half; };
+    const uint32_t chunk_off = (uint32_t)((ckey & 15) * D + cch * 8) * (INT8 ? 1 : 2);
+    // Block-table entries of a tile's halves (raw: scalar loads, looked up a phase before use).
+    // NH = 1: only this wave's half (its chunks lie in one, and there are no scales to find).
+    constexpr int NH = NC == 2 || INT8 ? 2 : 1, EB = INT8 ? 1 : 2;
+    struct Pages {
+        int pg[NH];
+    };
+    auto half_pos = [&](int kt, int x) { return kt * KT + 16 * (NH == 2 ? x : wave_half); };
+    auto pages_at = [&](int kt) {
+        Pages r;
+#pragma unroll
+        for (int x = 0; x < NH; x++) r.pg[x] = sload(bt, min(half_pos(kt, x) >> p.pshift, p.bt_stride - 1));
+        return r;
+    };
+    // Without key splits the first tiles' entries do not depend on the sequence's position:
+    // their loads go out together with those of the query counts.
+    Pages rp[4];
+    auto first_pages = [&](int lo) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) rp[j] = pages_at(KS ? lo + 2 * j + team : lo + j);
+    };
+    if (p.splits == 1) first_pages(0);
     const int tok0 = p.qsl ? sload(p.qsl, b) : b * p.nmax;
     const int nb = p.qsl ? min(sload(p.qsl, b + 1) - tok0, p.nmax) : p.nmax;   // at most max_query_len
-    const int start = max(sload(p.positions, nb > 0 ? tok0 : 0), 0), len = start + nb;   // a negative position reads as 0
     const int t_first = qt * p.TQ;
     if (t_first >= nb) return;
+    const int start = max(sload(p.positions, tok0), 0), len = start + nb;   // a negative position reads as 0
     const int t_last = min(t_first + p.TQ, nb) - 1;
     const int kend = p.causal ? start + t_last + 1 : len;
     const int nkt = (kend + KT - 1) / KT;
     const int per = (nkt + p.splits - 1) / p.splits;
     const int kt_lo = min(split * per, nkt), kt_hi = min(kt_lo + per, nkt);
-    const int N = kt_hi - kt_lo;                   // key tiles of this work-group
+    const int N = KS ? (kt_hi - kt_lo + 1) / 2 : kt_hi - kt_lo;   // steps of this work-group
     const size_t unit = ((size_t)b * p.Hk + h) * p.splits + split;
-    const int32_t *bt = p.bt + (size_t)b * p.bt_stride;
     const int mask_from = p.causal ? start + t_first : len - 1;
     if (N == 0) {
         // A split with no keys: neutral partials (m = -big, l = 0, acc = 0).
-        for (int idx = tid; idx < ROWS * (D + 2); idx += 64 * NW) {
+        for (int idx = tid; idx < RW * (D + 2); idx += 64 * NW) {
             const int rr = idx / (D + 2), c = idx - rr * (D + 2);
             const int ttl = rr / p.G, gg = rr - ttl * p.G, tt = t_first + ttl;
             if (ttl < p.TQ && tt < nb)
@@ -117,81 +186,139 @@ __global__ void __launch_bounds__(64 * NW) prefill_pp_kernel(PPParams p) {
         return;
     }
 
-    // This thread's staging chunk of every tile: key ckey (team A: 0-15, team B: 16-31),
-    // 16-byte chunk cch of the head dimension.
-    const int ckey = tid >> 4, cch = tid & 15;
-    const int half = team;                         // == ckey >> 4, wave-uniform
-    const long long chunk_off = (long long)(ckey & 15) * D + cch * 8;
+    // Key tile of step j (this team's, KS; its odd tile out is masked by position).
+    auto tile = [&](int j) { return KS ? kt_lo + 2 * j + team : kt_lo + j; };
 
-    // This wave's half of tile j (clamped to the last tile, so loads past the end re-read
-    // it and are never stored): its block-table entry (raw_half, a scalar load, looked up a
-    // step before use so its wait does not fall right after it) and its row base in
-    // elements (half_base: page clamped into the pool, 32-bit page stride and head offset).
-    const uint32_t pstride = (uint32_t)p.Hk * p.P * D, hoff = (uint32_t)h * p.P * D;
-    auto half_pos = [&](int j) { return (kt_lo + min(j, N - 1)) * KT + 16 * half; };
-    auto raw_half = [&](int j) { return sload(bt, min(half_pos(j) >> p.pshift, p.bt_stride - 1)); };
-    auto half_base = [&](int raw, int j) -> long long {
-        return (long long)((uint64_t)(uint32_t)clamp_page(raw, p.num_pages) * pstride + hoff +
-                           (uint32_t)((half_pos(j) & (p.P - 1)) * D));
+    // Row offsets of a tile's halves in bytes from the KV head's first row (page clamped into
+    // the pool; an entry of 0 or less wraps and reads the last page). Tiles past the last are
+    // loaded from whatever page the table's next entries name, never used.
+    struct Bases {
+        uint64_t e[NH];
     };
+    const uint32_t pstride = (uint32_t)p.Hk * p.P * D * EB;
+    const size_t hoff = (size_t)h * p.P * D * EB, half_q = (size_t)p.num_pages * p.Hk * p.P * D;
+    const char *kbase = (INT8 ? (const char *)p.lq : (const char *)p.kp) + hoff;
+    const char *vbase_g = INT8 ? kbase + half_q : (const char *)p.vp + hoff;
+    auto bases = [&](const Pages &r, int j) {
+        Bases o;
+#pragma unroll
+        for (int x = 0; x < NH; x++)
+            o.e[x] = (uint64_t)min((uint32_t)(r.pg[x] - 1), (uint32_t)p.num_pages - 1) * pstride +
+                     (uint32_t)((half_pos(tile(j), x) & (p.P - 1)) * (D * EB));
+        return o;
+    };
+    auto base_of = [&](const Bases &o, int u) { return NH == 2 && half_of(u) ? o.e[NH - 1] : o.e[0]; };
 
-    struct Stage {
-        u32x4 k, v;
+    // a scalar base plus a per-lane 32-bit offset (scalar-base addressing)
+    auto chunk_at = [&](const char *base, uint64_t off) {
+        const uint64_t a = (uint64_t)base + off;
+        const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
+        const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+        typedef const __attribute__((address_space(1))) char *global_ptr;
+        return *(const __attribute__((address_space(1))) Chunk *)((global_ptr)((hi << 32) | lo) + chunk_off);
     };
-    Stage st[NBUF];
-    auto load = [&](Stage &s, long long base) {
-        s.k = *reinterpret_cast<const u32x4 *>(p.kp + base + chunk_off);
-        s.v = *reinterpret_cast<const u32x4 *>(p.vp + base + chunk_off);
+    const size_t half_s = (size_t)p.num_pages * p.Hk * p.P;
+    Chunk sk[2][NC], sv[LV][NC];                   // staged chunks
+    float ss[2];                                   // INT8: staged scale of key lane % 32 (keys', then values')
+    auto load_k = [&](Chunk &r, const Bases &o, int u) { r = chunk_at(kbase, base_of(o, u)); };
+    auto load_v = [&](Chunk &r, const Bases &o, int u) { r = chunk_at(vbase_g, base_of(o, u)); };
+    const float *sbase = p.ls + (size_t)h * p.P + (kg ? half_s : 0) + (r32 & 15);
+    auto load_s = [&](float &r, const Bases &o) {
+        // every wave loads the same 64 scales (no branch: the count of loads in flight stays
+        // static), one wave of the staging threads stores them
+        r = sbase[(r32 >> 4 ? o.e[NH - 1] : o.e[0]) / D];
     };
-    auto store_k = [&](const Stage &s, int buf) {
-        *reinterpret_cast<u32x4 *>(&sm.k[buf][ckey * KROW + cch * 8]) = s.k;
+    auto bf16_chunk = [&](const Chunk &r) -> u32x4 {
+        if constexpr (INT8) {
+            u32x4 o;
+            uint32_t a, b2, c, d;
+            i8x4_to_bf16(r[0], a, b2);
+            i8x4_to_bf16(r[1], c, d);
+            o[0] = a, o[1] = b2, o[2] = c, o[3] = d;
+            return o;
+        } else {
+            return r;
+        }
     };
-    auto store_v = [&](const Stage &s, int buf, int j) {
+    auto store_k = [&](const Chunk &r, int buf, int u) {
+        *reinterpret_cast<u32x4 *>(&sm.k[buf][(ckey + KPU * u) * KROW + cch * 8]) = bf16_chunk(r);
+    };
+    auto store_v = [&](const Chunk &r, int buf, int j, int u) {
         // Keys past kend in the last tile may hold any bits (even NaN) of an allocated
         // page: their probabilities are 0 and their values must be finite. Branch-free,
         // so the stage registers are never rewritten while loads are pending.
-        const uint32_t keep = (kt_lo + j) * KT + ckey < kend ? ~0u : 0u;
-        *reinterpret_cast<u32x4 *>(&sm.v[buf][ckey * VROW + cch * 8]) = s.v & keep;
+        const uint32_t keep = tile(j) * KT + ckey + KPU * u < kend ? ~0u : 0u;
+        *reinterpret_cast<u32x4 *>(&sm.v[buf][(ckey + KPU * u) * VROW + cch * 8]) = bf16_chunk(r) & keep;
+    };
+    const float smul = kg ? 1.0f : p.scale_log2;
+    auto store_s = [&](float r, int j) {
+        // scales of keys past kend may hold any bits too: zero
+        if (w == (KS ? 4 * team : 0)) sm.s[j & 3][lane] = tile(j) * KT + r32 < kend ? r * smul : 0.0f;
     };
 
-    // Query rows (B operand of S^T = K Q^T): wave w holds rows 32 w .. 32 w + 31.
-    const int r = w * 32 + r32, tl = r / p.G, g = r - tl * p.G, t = t_first + tl;
+    // Query rows (B operand of S^T = K Q^T): wave w holds rows 32 w .. 32 w + 31 (KS: both
+    // teams hold the same 128).
+    const int r = (KS ? w & 3 : w) * 32 + r32, tl = r / p.G, g = r - tl * p.G, t = t_first + tl;
     const bool row_ok = tl < p.TQ && t < nb;
-    const int qpos = p.causal && row_ok ? start + t : len - 1;
+    // last visible key of the row (KS: of this split too, whose odd tile out is masked by it)
+    const int qpos = min(p.causal && row_ok ? start + t : len - 1, kt_hi * KT - 1);
+
+    // Prologue: K of tiles 0 and 1 in LDS; K of tiles 2, 3 and V of tiles 0 .. LV - 1 in
+    // flight (in the order of their stores, so the waits before each store count exactly the
+    // younger loads).
+    Bases bs[4];                                   // bases of tiles i + 1 .. i + 3 in 1 .. 3
+    Pages raw4;                                    // block-table entries of tile i + 4
     bf16x8 qreg[NQB];
     {
-        const uint16_t *qr = p.q + ((size_t)(tok0 + (row_ok ? t : 0)) * p.Hq + h * p.G + g) * D;
+        if (p.splits != 1) first_pages(kt_lo);
 #pragma unroll
-        for (int i = 0; i < NQB; i++)
-            qreg[i] = row_ok ? as_bf16x8(*reinterpret_cast<const u32x4 *>(qr + i * 16 + kg * 8))
-                             : as_bf16x8((u32x4){0u, 0u, 0u, 0u});
+        for (int j = 0; j < 4; j++) bs[j] = bases(rp[j], j);
+        Chunk k0[NC], k1[NC];
+        float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+        for (int u = 0; u < NC; u++) load_k(k0[u], bs[0], u);
+        if constexpr (INT8) load_s(s0, bs[0]);
+#pragma unroll
+        for (int u = 0; u < NC; u++) load_k(k1[u], bs[1], u);
+        if constexpr (INT8) load_s(s1, bs[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint16_t *qr = p.q + ((size_t)(tok0 + (row_ok ? t : 0)) * p.Hq + h * p.G + (row_ok ? g : 0)) * D;
+        u32x4 raw[NQB];
+#pragma unroll
+        for (int i = 0; i < NQB; i++) raw[i] = *reinterpret_cast<const u32x4 *>(qr + i * 16 + kg * 8);
+#pragma unroll
+        for (int x = 0; x < 2; x++) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (x < LV) {
+#pragma unroll
+                for (int u = 0; u < NC; u++) load_v(sv[x % LV][u], bs[x], u);
+            }
+#pragma unroll
+            for (int u = 0; u < NC; u++) load_k(sk[x][u], bs[2 + x], u);
+            if constexpr (INT8) load_s(ss[x], bs[2 + x]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        raw4 = pages_at(tile(4));
+#pragma unroll
+        for (int u = 0; u < NC; u++) store_k(k0[u], 0, u);
+        if constexpr (INT8) store_s(s0, 0);
+#pragma unroll
+        for (int u = 0; u < NC; u++) store_k(k1[u], 1, u);
+        if constexpr (INT8) store_s(s1, 1);
+        const uint32_t keep = row_ok ? ~0u : 0u;
+#pragma unroll
+        for (int i = 0; i < NQB; i++) {
+            if constexpr (INT8) {
+                // bf16(q * smooth) (attention.jl:90-95)
+                const int d0 = i * 16 + kg * 8;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    raw[i][e] = pack_bf16x2(__uint_as_float(raw[i][e] << 16) * p.smooth[d0 + 2 * e],
+                                            __uint_as_float(raw[i][e] & 0xffff0000u) * p.smooth[d0 + 2 * e + 1]);
+            }
+            qreg[i] = as_bf16x8(raw[i] & keep);
+        }
     }
-
-    // Prologue: tiles 0-2 in flight; tile 0's K and V and tile 1's K in LDS; tile 3 in
-    // flight in stage 0.
-    // (Scheduling fences keep the loads in tile order, so the waits before each LDS
-    // store count exactly the younger tiles still in flight.)
-    int r0 = raw_half(0), r1 = raw_half(1), r2 = raw_half(2), r3 = raw_half(3);
-    long long nbase = half_base(r0, 0);
-    load(st[0], nbase);
-    nbase = half_base(r1, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    load(st[1], nbase);
-    nbase = half_base(r2, 2);
-    __builtin_amdgcn_sched_barrier(0);
-    load(st[2], nbase);
-    nbase = half_base(r3, 3);
-    int nraw = raw_half(4);
-    __builtin_amdgcn_sched_barrier(0);
-    store_k(st[0], 0);
-    store_v(st[0], 0, 0);
-    // Unconditional (with one tile, tile 1 is a re-read of tile 0 that is never used):
-    // a branch here would let the compiler sink the next load into it and leave the
-    // loop with two different counts of loads in flight, which costs conservative waits.
-    store_k(st[1], 1);
-    load(st[0], nbase);
-    nbase = half_base(nraw, 4);
-    nraw = raw_half(5);
 
     f32x16 o[NDB];
 #pragma unroll
@@ -206,35 +333,46 @@ __global__ void __launch_bounds__(64 * NW) prefill_pp_kernel(PPParams p) {
     const int c16 = lane >> 4, s16 = lane & 15;
     const int tr_row = 4 * (c16 >> 1) + (s16 >> 2), tr_col = 16 * (c16 & 1) + 4 * (s16 & 3);
 
-    // O^T += V^T P^T for the tile in V buffer vb.
-    auto pv = [&](int vb) {
-        const uint16_t *vbase = &sm.v[vb][tr_row * VROW + tr_col];
-#pragma unroll
-        for (int db = 0; db < NDB; db++)
-#pragma unroll
-            for (int hh = 0; hh < 2; hh++) {
-                const u32x2 lo = lds_tr16(vbase + (16 * hh) * VROW + 32 * db);
-                const u32x2 hi = lds_tr16(vbase + (16 * hh + 8) * VROW + 32 * db);
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8((u32x4){lo[0], lo[1], hi[0], hi[1]}),
-                                                               pb[hh], o[db], 0, 0, 0);
-            }
+    u32x4 ka[NQB];                     // K operands of the next score product
+    u32x2 va[2 * NDB][2];              // V^T operands of the value product
+    auto read_k = [&](int kb, int i) {
+        ka[i] = *reinterpret_cast<const u32x4 *>(&sm.k[kb][r32 * KROW + kg * 8] + i * 16);
     };
-    // S^T = K Q^T for the tile in K buffer kb (one accumulation chain: dependent MFMAs
-    // issue back to back).
-    auto qk = [&](int kb) {
-#pragma unroll
-        for (int e = 0; e < 16; e++) sc[e] = 0.0f;
-        const uint16_t *krow = &sm.k[kb][r32 * KROW + kg * 8];
-#pragma unroll
-        for (int i = 0; i < NQB; i++)
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(*reinterpret_cast<const u32x4 *>(krow + i * 16)),
-                                                         qreg[i], sc, 0, 0, 0);
+    // value MFMA x: keys 16 (x / NDB) .. + 15, output block x % NDB
+    auto read_v = [&](int vb, int x) {
+        const uint16_t *vbase = &sm.v[vb][tr_row * VROW + tr_col] + 16 * (x / NDB) * VROW + 32 * (x % NDB);
+        va[x][0] = lds_tr16(vbase);
+        va[x][1] = lds_tr16(vbase + 8 * VROW);
     };
-    // Online softmax of tile j's scores (exp2 domain, lazy rescale) -> pb. Only tiles
+    auto pv = [&](int x) {
+        o[x % NDB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            as_bf16x8((u32x4){va[x][0][0], va[x][0][1], va[x][1][0], va[x][1][1]}), pb[x / NDB], o[x % NDB], 0, 0, 0);
+    };
+    auto qk = [&](int i) {
+        if (i == 0) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) sc[e] = 0.0f;
+        }
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(ka[i]), qreg[i], sc, 0, 0, 0);
+    };
+    // Online softmax of step j's scores (exp2 domain, lazy rescale) -> pb. Only tiles
     // reaching past mask_from (the diagonal / last tiles) compare key positions.
-    auto softmax = [&](int j, auto need_mask) {
-        const int kt = kt_lo + j;
-        if (need_mask) {
+    const int jm = min(mask_from + 1, kt_hi * KT); // first key position that a row may not see
+    auto softmax = [&](int j) {
+        const int kt = tile(j);
+        f32x4 svq[4];
+        if constexpr (INT8) {
+            // a lane's scores are of keys 8 (e / 4) + 4 kg + e % 4
+            const float *sp = &sm.s[j & 3][4 * kg];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const f32x4 skq = *reinterpret_cast<const f32x4 *>(sp + 8 * q);
+                svq[q] = *reinterpret_cast<const f32x4 *>(sp + KT + 8 * q);
+#pragma unroll
+                for (int e = 0; e < 4; e++) sc[4 * q + e] *= skq[e];   // scaled to log2 units too
+            }
+        }
+        if (kt * KT + KT > jm) {
             // A real branch (the empty asm keeps the compiler from if-converting the
             // selects into every tile): key 8 (e / 4) + 4 kg + e % 4 is visible iff
             // it is <= qpos - kt * KT.
@@ -244,14 +382,10 @@ __global__ void __launch_bounds__(64 * NW) prefill_pp_kernel(PPParams p) {
             for (int e = 0; e < 16; e++)
                 sc[e] = 8 * (e >> 2) + (e & 3) <= lim ? sc[e] : -INFINITY;
         }
-        float x[16];
         float mt = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 16; e++) {
-            x[e] = sc[e];
-            mt = fmaxf(mt, x[e]);
-        }
-        mt *= p.scale_log2;
+        for (int e = 0; e < 16; e++) mt = fmaxf(mt, sc[e]);
+        if constexpr (!INT8) mt *= p.scale_log2;
         if (__any(mt > m + RESCALE_LOG2)) {
             mt = fmaxf(mt, __shfl_xor(mt, 32));
             const float mn = fmaxf(m, mt);
@@ -264,8 +398,9 @@ __global__ void __launch_bounds__(64 * NW) prefill_pp_kernel(PPParams p) {
         float pe[16], ps = 0.0f;
 #pragma unroll
         for (int e = 0; e < 16; e++) {
-            pe[e] = fast_exp2(__builtin_fmaf(x[e], p.scale_log2, -m));
+            pe[e] = fast_exp2(INT8 ? sc[e] - m : __builtin_fmaf(sc[e], p.scale_log2, -m));
             ps += pe[e];
+            if constexpr (INT8) pe[e] *= svq[e >> 2][e & 3];
         }
         l += ps;
 #pragma unroll
@@ -281,72 +416,234 @@ __global__ void __launch_bounds__(64 * NW) prefill_pp_kernel(PPParams p) {
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
     };
-    // One step i (ring slot S = i % 3): phase X_i, barrier, phase Y_i, barrier.
-    auto step = [&](int i, auto slot, auto need_mask) {
-        constexpr int S = decltype(slot)::value;
-        constexpr int S1 = (S + 1) % NBUF, S2 = (S + 2) % NBUF;
-        qk(S);
-        if (i > 0) pv(S2);                           // tile i - 1
-        phase_barrier();
-        softmax(i, need_mask);
-        if (i + 2 < N) store_k(st[S2], S2);          // tile i + 2 (loaded at step i - 2)
-        if (i + 1 < N) store_v(st[S1], S1, i + 1);   // tile i + 1 (loaded at step i - 3)
-        load(st[S1], nbase);                         // tile i + 4
-        nbase = half_base(nraw, i + 5);
-        nraw = raw_half(i + 6);
-        phase_barrier();
+    // Phase X_i (S = i % 2; FIRST: i = 0, no values yet). MFMAs: three scores, then values and
+    // scores in turn (independent accumulators), then the values left. The gaps between them
+    // (32 cycles each, about five instructions) take the side operations: value operands of
+    // tile i - 1; V(i) and K(i + 2) into LDS (loaded LV and 2 steps before); the offsets of
+    // tile i + 4; the staging registers' next loads; key operands of tile i + 1 (a key
+    // operand's register is free once its score MFMA has issued). gap_of: the MFMA after which
+    // operation X is issued, for 16 MFMAs (D = 128), halved for D = 64.
+    auto phase_x = [&](int i, auto slot, auto first) {
+        constexpr int S = decltype(slot)::value, S1 = 1 - S, SV = S % LV;
+        constexpr bool FIRST = decltype(first)::value;
+        constexpr int NM = NQB + 2 * NDB, SC = INT8 ? 1 : 0;
+        constexpr int O_SV = 2 * NDB, O_SK = O_SV + NC, O_SS = O_SK + NC, O_BA = O_SS + SC, O_LV = O_BA + NH,
+                      O_LK = O_LV + NC, O_LS = O_LK + NC, O_RK = O_LS + SC, NS = O_RK + NQB;
+        constexpr auto gap_of = [](int X) {
+            const int g = X < O_SV   ? X * 8 / O_SV / 2
+                          : X < O_SK ? 4 + (X - O_SV)
+                          : X < O_SS ? (NC == 2 ? 6 : 5) + (X - O_SK)
+                          : X < O_BA ? 7
+                          : X < O_LV ? 7 + (X - O_BA)
+                          : X < O_LK ? 8 + (X - O_LV)
+                          : X < O_LS ? 9 + (X - O_LK)
+                          : X < O_RK ? 11
+                                     : 9 + (X - O_RK) * 8 / NQB / 2;
+            return g * NM / 16;
+        };
+        Bases b4;
+        unroll<NM>([&](auto mi) {
+            constexpr int M = decltype(mi)::value;
+            constexpr int T = M - 3;               // after the first three scores
+            constexpr bool IS_QK = M < 3 || (T / 2 < NQB - 3 && T % 2 == 1);
+            if constexpr (IS_QK) qk(M < 3 ? M : 3 + T / 2);
+            else if constexpr (!FIRST) pv(T / 2 < NQB - 3 ? T / 2 : T - (NQB - 3));
+            unroll<NS>([&](auto xi) {
+                constexpr int X = decltype(xi)::value;
+                if constexpr (gap_of(X) == M) {
+                    if constexpr (X < O_SV) {
+                        if constexpr (!FIRST) read_v(S1, X);
+                    } else if constexpr (X < O_SK) {
+                        store_v(sv[SV][X - O_SV], S, i, X - O_SV);
+                    } else if constexpr (X < O_SS) {
+                        store_k(sk[S][X - O_SK], S, X - O_SK);
+                    } else if constexpr (X < O_BA) {
+                        store_s(ss[S], i + 2);
+                    } else if constexpr (X < O_LV) {
+                        b4.e[X - O_BA] = bases(raw4, i + 4).e[X - O_BA];
+                    } else if constexpr (X < O_LK) {
+                        load_v(sv[SV][X - O_LV], bs[LV], X - O_LV);
+                    } else if constexpr (X < O_LS) {
+                        load_k(sk[S][X - O_LK], b4, X - O_LK);
+                    } else if constexpr (X < O_RK) {
+                        load_s(ss[S], b4);
+                    } else {
+                        read_k(S1, X - O_RK);
+                    }
+                }
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        bs[1] = bs[2], bs[2] = bs[3], bs[3] = b4;
     };
-    // First tile (relative) whose keys reach past mask_from.
-    const int jm = max(0, (mask_from + 1) / KT - kt_lo);
-    auto step_m = [&](int i, auto slot) { step(i, slot, i >= jm); };
+    auto phase_y = [&](int i) {
+        raw4 = pages_at(tile(i + 5));
+        softmax(i);
+        // the lookup's wait falls here, where the barrier waits for LDS anyway
+        asm volatile("" : "+s"(raw4.pg[0]));
+        if constexpr (NH == 2) asm volatile("" : "+s"(raw4.pg[NH - 1]));
+    };
 
     phase_barrier();
-    if (team == 1) phase_barrier();                  // team B runs one phase behind
-    for (int i = 0; i < N; i += 3) {
-        step_m(i, IC<0>{});
-        if (i + 1 >= N) break;
-        step_m(i + 1, IC<1>{});
-        if (i + 2 >= N) break;
-        step_m(i + 2, IC<2>{});
+#pragma unroll
+    for (int q = 0; q < NQB; q++) read_k(0, q);
+    phase_barrier();                               // X_0 overwrites tile 0's keys
+    if (!SOLO && team == 1) phase_barrier();       // team B runs one phase behind
+    // SOLO: one barrier a step
+    auto x_barrier = [&] {
+        if constexpr (!SOLO) phase_barrier();
+        else __builtin_amdgcn_sched_barrier(0);
+    };
+    phase_x(0, IC<0>{}, std::true_type{});
+    x_barrier();
+    // Whole pairs of steps, then the last one or two: a loop with one exit keeps the count of
+    // loads in flight static, so the waits before the LDS stores leave the younger ones pending.
+    int i = 0;
+    for (; i + 2 < N; i += 2) {
+        phase_y(i);
+        phase_barrier();
+        phase_x(i + 1, IC<1>{}, std::false_type{});
+        x_barrier();
+        phase_y(i + 1);
+        phase_barrier();
+        phase_x(i + 2, IC<0>{}, std::false_type{});
+        x_barrier();
     }
-    pv((N - 1) % NBUF);                              // last tile's PV
-    if (team == 0) phase_barrier();
+    phase_y(i);
+    phase_barrier();
+    if (i + 1 < N) {
+        phase_x(i + 1, IC<1>{}, std::false_type{});
+        x_barrier();
+        phase_y(i + 1);
+        phase_barrier();
+    }
+    // last tile's values
+#pragma unroll
+    for (int x = 0; x < 2 * NDB; x++) read_v((N - 1) & 1, x);
+#pragma unroll
+    for (int x = 0; x < 2 * NDB; x++) pv(x);
+    if (!SOLO && team == 0) phase_barrier();
 
     l += __shfl_xor(l, 32);
+    // The output blocks this wave writes: all of them, or (KS) half of them after the teams'
+    // states are merged: each wave hands the other team's wave of its rows (same rows, same
+    // lane layout) the half it does not write.
+    int db0 = 0;
+    constexpr int NOUT = KS ? NDB / 2 : NDB;
+    if constexpr (KS) {
+        f32x4 *slab = reinterpret_cast<f32x4 *>(smem_raw);
+        float2 *ml = reinterpret_cast<float2 *>(smem_raw + NW * 64 * NOUT * 64);
+        __syncthreads();                           // every wave is done with the tiles
+        auto give = [&](int d0) {
+#pragma unroll
+            for (int x = 0; x < NOUT; x++)
+#pragma unroll
+                for (int e4 = 0; e4 < 4; e4++)
+                    slab[(w * NOUT * 4 + 4 * x + e4) * 64 + lane] =
+                        (f32x4){o[d0 + x][4 * e4], o[d0 + x][4 * e4 + 1], o[d0 + x][4 * e4 + 2], o[d0 + x][4 * e4 + 3]};
+        };
+        if (team == 0) give(NOUT);
+        else give(0);
+        ml[w * 64 + lane] = make_float2(m, l);
+        __syncthreads();
+        const int ow = w ^ 4;
+        const float2 oml = ml[ow * 64 + lane];
+        const float mx = fmaxf(m, oml.x), wa = fast_exp2(m - mx), wb = fast_exp2(oml.x - mx);
+        auto take = [&](int d0) {
+#pragma unroll
+            for (int x = 0; x < NOUT; x++)
+#pragma unroll
+                for (int e4 = 0; e4 < 4; e4++) {
+                    const f32x4 v = slab[(ow * NOUT * 4 + 4 * x + e4) * 64 + lane];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[x][4 * e4 + e] = o[d0 + x][4 * e4 + e] * wa + v[e] * wb;
+                }
+        };
+        if (team == 0) take(0);
+        else take(NOUT);
+        m = mx;
+        l = l * wa + oml.y * wb;
+        db0 = team * NOUT;
+    }
     if (!row_ok) return;
     if (p.splits > 1) {
         float *dst = p.part + (unit * p.M + (size_t)t * p.G + g) * (D + 2);
 #pragma unroll
-        for (int db = 0; db < NDB; db++)
+        for (int db = 0; db < NOUT; db++)
 #pragma unroll
             for (int e4 = 0; e4 < 4; e4++)
-                *reinterpret_cast<f32x4 *>(dst + 32 * db + 8 * e4 + 4 * kg) =
+                *reinterpret_cast<f32x4 *>(dst + 32 * (db0 + db) + 8 * e4 + 4 * kg) =
                     (f32x4){o[db][4 * e4], o[db][4 * e4 + 1], o[db][4 * e4 + 2], o[db][4 * e4 + 3]};
-        if (kg == 0) *reinterpret_cast<float2 *>(dst + D) = make_float2(m, l);
+        if (kg == 0 && db0 == 0) *reinterpret_cast<float2 *>(dst + D) = make_float2(m, l);
         return;
     }
     const float inv = 1.0f / l;
     uint16_t *orow = p.out + ((size_t)(tok0 + t) * p.Hq + h * p.G + g) * D;
 #pragma unroll
-    for (int db = 0; db < NDB; db++)
+    for (int db = 0; db < NOUT; db++)
 #pragma unroll
         for (int e4 = 0; e4 < 4; e4++) {
-            const int d = 32 * db + 8 * e4 + 4 * kg;
+            const int d = 32 * (db0 + db) + 8 * e4 + 4 * kg;
             const uint32_t w0 = pack_bf16x2(o[db][4 * e4 + 0] * inv, o[db][4 * e4 + 1] * inv);
             const uint32_t w1 = pack_bf16x2(o[db][4 * e4 + 2] * inv, o[db][4 * e4 + 3] * inv);
             *reinterpret_cast<u32x2 *>(orow + d) = (u32x2){w0, w1};
         }
 }
 
+template <int D, bool INT8, int FORM>
+void launch_pp(const PPParams &p, int B, hipStream_t s) {
+    prefill_pp_kernel<D, INT8, FORM><<<dim3(p.Hk, p.qtiles * p.splits, B), FORM == TI_PP_SOLO ? 256 : 512, 0, s>>>(p);
+}
+
+template <int D, bool INT8>
+void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
+    if constexpr (D == 128 && !INT8) {
+        if (form == TI_PP_SHARED) return launch_pp<D, INT8, TI_PP_SHARED>(p, B, s);
+    }
+    if (form == TI_PP_SOLO) launch_pp<D, INT8, TI_PP_SOLO>(p, B, s);
+    else launch_pp<D, INT8, TI_PP_KSPLIT>(p, B, s);
+}
+
 }  // namespace
 
-// The ping-pong kernel takes dense bf16 caches with head_dim 128, power-of-two pages of at
-// least 16 tokens and G dividing 256 (each work-group holds 256 packed rows).
-bool ti_prefill_pp_eligible(const ti_attention_args *a, const ti_kv_cache *c) {
-    const int G = a->q_heads / c->kv_heads;
-    const int P = c->page_size;
-    return c->kind == TI_KV_DENSE && a->dtype == TI_BF16 && c->head_dim == D && P >= 16 &&
-           (P & (P - 1)) == 0 && ROWS % G == 0;
+// The ping-pong kernel takes bf16 activations over dense or INT8 caches with head_dim 64 or
+// 128, power-of-two pages of at least 16 tokens (a page of all KV heads under 4 GiB: 32-bit
+// strides) and at most 128 heads per KV head.
+//
+// The library's pick counts the launch's 128-row work-groups, W (head counts 32 / 8 unless
+// stated; each figure: this form against the kernel that takes the step otherwise, the
+// four-wave or the 16-row paired one, same process, graph replays, inputs warm):
+//   W <= 128: none. A work-group's fixed cost (about 7 us: first loads, merge, stores) and
+//     idle CUs outweigh the faster steps (512 tokens, W = 128: the 16-row kernel's one round of
+//     256 work-groups takes 9.3 us).
+//   W <= 512: KSPLIT. At most two work-groups per CU, one resident at a time, each with half
+//     the steps of an unsplit q-tile: 520 tokens 14.4 against 15.8 us, 1024 22.5 against
+//     26.1, 2048 47.2 against 56.5; 576 on 2000 40.7 against 65.2; D = 64, 1024 15.1 against
+//     21.4. INT8 tiles cost twice the staging there, and single prompts start later: 1024
+//     tokens (W = 256) 31.1 against 29.8, 1280 37.0 against 40.3. So do q-tiles with rows to
+//     spare (G = 3: 768 tokens, W = 152, 18.1 against 17.7).
+//   more: SHARED for dense D = 128 (half the loads and LDS stores per row): 3072 tokens 85.0
+//     against 118.7 us, 8192 493 against 539; else SOLO, whose work-groups share a CU (two,
+//     D = 64 three) and hide each other's fixed cost: INT8 3072 tokens 110.8 against 145.8,
+//     D = 64 8192 309 against 394, eight D = 64 prompts of 100 to 2000 tokens 58.8 against
+//     78.3. SOLO also takes dense batches of short sequences, whose 256-row tiles are mostly
+//     padding: 16 prompts of 30 to 300 tokens 22.1 us, SHARED 25.3, 28.2 before.
+//   At most two q-tiles per sequence (T <= 2): SOLO from W = 512 (32 x 60 tokens from scratch
+//     / on 2000: 0.76 / 0.84 of the time), KSPLIT at D = 128 dense (9 x 60: 0.75), INT8 from 256.
+int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path) {
+    const int G = a->q_heads / c->kv_heads, P = c->page_size, D = c->head_dim;
+    if (a->dtype != TI_BF16 || (D != 64 && D != 128) || P < 16 || (P & (P - 1)) || G > 128 ||
+        2ull * c->kv_heads * P * D > 0xffffffffull)
+        return TI_PP_NONE;
+    const bool dense = c->kind == TI_KV_DENSE, dense128 = dense && D == 128;
+    if (path == TI_PATH_PREFILL_PINGPONG && dense128) return TI_PP_SHARED;
+    if (path != TI_PATH_AUTO && path != TI_PATH_PREFILL) return TI_PP_NONE;
+    const long long TQ = 128 / G, T = (a->max_query_len + TQ - 1) / TQ, W = T * c->kv_heads * a->num_seqs;
+    if (T <= 2) return W >= 512 ? TI_PP_SOLO : (D == 128 && W >= (dense ? 129 : 256) ? TI_PP_KSPLIT : TI_PP_NONE);
+    const int first = dense ? (128 % G == 0 ? 129 : 160) : (a->num_seqs > 1 ? 160 : D == 64 ? 256 : 257);
+    if (W < first) return TI_PP_NONE;
+    if (W <= 512) return TI_PP_KSPLIT;
+    return dense128 && T > 6 && !(a->num_seqs >= 8 && W > 1024) ? TI_PP_SHARED : TI_PP_SOLO;
 }
 
 int ti_launch_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, const ti_prefill_plan &pl,
@@ -356,6 +653,9 @@ int ti_launch_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, const
     p.out = (uint16_t *)a->out;
     p.kp = (const uint16_t *)c->k_pages;
     p.vp = (const uint16_t *)c->v_pages;
+    p.lq = c->layer_q;
+    p.ls = c->layer_scale;
+    p.smooth = c->smooth;
     p.positions = a->positions;
     p.qsl = a->query_start_loc;
     p.bt = a->block_tables;
@@ -371,11 +671,18 @@ int ti_launch_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, const
     p.scale_log2 = a->scale * LOG2E;
     p.part = (float *)a->workspace;
     p.splits = pl.splits;
+    p.sshift = __builtin_ctz(pl.splits);
     p.M = pl.rows;
     p.TQ = pl.TQ;
     p.qtiles = pl.qtiles;
-    dim3 grid(c->kv_heads, p.qtiles * pl.splits, a->num_seqs);
-    prefill_pp_kernel<<<grid, 64 * NW, 0, s>>>(p);
+    const bool int8 = c->kind == TI_KV_INT8;
+    if (c->head_dim == 64) {
+        if (int8) launch_pp_form<64, true>(p, pl.pp, a->num_seqs, s);
+        else launch_pp_form<64, false>(p, pl.pp, a->num_seqs, s);
+    } else {
+        if (int8) launch_pp_form<128, true>(p, pl.pp, a->num_seqs, s);
+        else launch_pp_form<128, false>(p, pl.pp, a->num_seqs, s);
+    }
     if (hipGetLastError() != hipSuccess) return TI_ERR_LAUNCH;
     return pl.splits > 1 ? ti_launch_combine(a, c, pl.rows, pl.splits, s) : TI_OK;
 }
