@@ -255,3 +255,52 @@ def test_attention_inputs_out_of_range(gpu, D, int8):
         orc.attention_inputs(qkv[:1], None, None, cs_tab, positions[:1], slots[:1], nq, nkv, 1e-6, True,
                              k_pages=rkp, v_pages=rvp)
         assert np.array_equal(host(kp), rkp) and np.array_equal(host(vp), rvp)
+
+
+# (dtype, INT8 cache, D, heads, kv_heads, tokens): both sides of the 256-token rule of the fused
+# kernel's lane layout, head counts that fill its waves or not, tokens that take two work-groups.
+LAYOUT_CASES = [(True, False, 128, 32, 8, 255), (True, False, 128, 32, 8, 256), (True, False, 128, 32, 4, 300),
+                (True, False, 128, 64, 8, 257), (True, False, 128, 3, 1, 256), (True, False, 64, 24, 8, 256),
+                (True, False, 64, 5, 5, 301), (True, False, 64, 96, 8, 255), (True, True, 128, 32, 8, 256),
+                (True, True, 64, 32, 4, 270), (False, False, 128, 16, 8, 256), (False, True, 64, 12, 4, 3)]
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("case", LAYOUT_CASES, ids=str)
+def test_attention_inputs_layouts(gpu, case, norm):
+    """Bit-identical to rmsnorm_ -> rope_ -> store_kv_, whatever layout the fused kernel takes;
+    tokens at positions outside the table and at slots outside the pool write nothing."""
+    bf16, int8, D, nq, nkv, n = case
+    P, L, eps = 16, 512, 1e-6
+    pages = n // P + 2
+    g = rng(4700 + n + D + nq + int8)
+    _, _, table = _table(g, D, L, bf16)
+    positions = g.integers(0, L, n).astype(np.int32)
+    slots = (g.permutation(pages * P)[:n] + 1).astype(np.int32)
+    positions[n // 2], slots[n // 3] = L, pages * P + 1
+    pos_d, slots_d = torch.from_numpy(positions).cuda(), torch.from_numpy(slots).cuda()
+    qkv = dev(randn(g, n, nq + 2 * nkv, D, bf16=bf16), bf16)
+    qn, kn = (dev(randn(g, D, bf16=bf16), bf16), dev(randn(g, D, bf16=bf16), bf16)) if norm else (None, None)
+    cs = torch.from_numpy(smoothing(g, D))
+
+    def pools():
+        if int8:
+            k, v = ti.int8_kv_pools(D, P, nkv, pages, key_smoothing=cs)
+            return (k, v), (k.layer_q, k.layer_scale)
+        k = torch.zeros((pages, nkv, P, D), dtype=DT[bf16], device="cuda")
+        return (k, torch.zeros_like(k)), None
+
+    (k, v), flat = pools()
+    q = torch.zeros((n, nq, D), dtype=DT[bf16], device="cuda")
+    ti.attention_inputs_(BE, q, k, v, qkv, qn, kn, table, pos_d, slots_d, eps)
+    (k2, v2), flat2 = pools()
+    qs, kk, vv = qkv[:, :nq].contiguous(), qkv[:, nq:nq + nkv].contiguous(), qkv[:, nq + nkv:].contiguous()
+    if norm:
+        qs, kk = ti.rmsnorm(BE, qs, qn, eps), ti.rmsnorm(BE, kk, kn, eps)
+    q2 = ti.rope_(BE, torch.zeros_like(qs), qs, table.cos, table.sin, pos_d)
+    keep = slots_d.clone()
+    keep[n // 2] = 0                                 # the fused op skips a token outside the table
+    ti.store_kv_(BE, k2, v2, ti.rope(BE, kk, table.cos, table.sin, pos_d), vv, keep)
+    assert torch.equal(q, q2)
+    for x, y in zip(flat or (k, v), flat2 or (k2, v2)):
+        assert torch.equal(x, y)

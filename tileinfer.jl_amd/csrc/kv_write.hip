@@ -17,7 +17,8 @@ namespace {
 __device__ __forceinline__ long long slot_row(int32_t slot, int h, int P, int H, int pages) {
     long long s = (long long)slot - 1;
     if (s < 0 || s >= (long long)P * pages) return -1;
-    return (s % P) + (long long)P * h + (long long)P * H * (s / P);
+    const uint32_t s32 = (uint32_t)s, page = s32 / (uint32_t)P;   // 32-bit division: a slot is an int32
+    return (long long)(s32 - page * (uint32_t)P) + (long long)P * h + (long long)P * H * page;
 }
 
 // ---- rope (src/ops/tile/elementwise.jl:10-27; reference src/ops/reference.jl:32-39) ----
@@ -249,36 +250,35 @@ __global__ void __launch_bounds__(64) attention_inputs_kernel(
     }
 }
 
-// quantize_store for one vector held by an LPH-lane group, 8 elements per lane: elements
-// x[0..3] go to bytes o1 .. o1 + 3 of the row, x[4..7] to o2 .. o2 + 3 (as 32-bit words).
-template <int LPH>
-__device__ __forceinline__ void quantize_group(const float (&x)[8], int8_t *__restrict__ qrow, int o1,
+// quantize_store for one vector held by an LPH-lane group, N elements per lane: the first
+// half of x goes to bytes o1 .. of the row, the second to o2 .. (as 32-bit words).
+template <int LPH, int N>
+__device__ __forceinline__ void quantize_group(const float (&x)[N], int8_t *__restrict__ qrow, int o1,
                                                int o2, float *__restrict__ scale, int u) {
     float m = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 8; e++) m = fmaxf(m, fabsf(x[e]));
+    for (int e = 0; e < N; e++) m = fmaxf(m, fabsf(x[e]));
 #pragma unroll
     for (int o = LPH / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
     const float inv = m > 0.0f ? __fdiv_rn(127.0f, m) : 0.0f;
-    uint32_t w[2] = {0u, 0u};
+    constexpr int NW = N / 8;   // words per half
+    uint32_t w[2 * NW];
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
+    for (int i = 0; i < 2 * NW; i++) w[i] = 0u;
+#pragma unroll
+    for (int e = 0; e < N; e++) {
         const int qv = (int)floorf(__fadd_rn(__fmul_rn(x[e], inv), 0.5f));
         w[e >> 2] |= (uint32_t)(uint8_t)(int8_t)qv << (8 * (e & 3));
     }
-    *reinterpret_cast<uint32_t *>(qrow + o1) = w[0];
-    *reinterpret_cast<uint32_t *>(qrow + o2) = w[1];
+#pragma unroll
+    for (int i = 0; i < NW; i++) {
+        reinterpret_cast<uint32_t *>(qrow + o1)[i] = w[i];
+        reinterpret_cast<uint32_t *>(qrow + o2)[i] = w[NW + i];
+    }
     if (u == 0) *scale = __fdiv_rn(m, 127.0f);
 }
 
-// Vectorized form of attention_inputs_kernel for head_dim 128 or 64: D / 8 lanes per head
-// (16 or 8), lane u owning elements 4u .. 4u + 3 of each half (8-byte bf16 / 16-byte Float32
-// loads), 2048 / D heads per 256-thread work-group: grid (n, ceil((nq + nkv) / (2048 / D))).
-// Same rounding points element by element. With the q/k norm, each lane keeps the four
-// per-lane partials a_i^2 + b_i^2 (i = 4u + e) that the one-wave kernel's lanes hold and
-// combines them in that kernel's butterfly order (xor 32, 16, 8, 4 across lanes u ^ 8,
-// u ^ 4, u ^ 2, u ^ 1, then xor 2 and 1 inside the lane), so the sum of squares, and with
-// it every output, is bit-identical to the one-wave kernel and to rmsnorm_kernel.
+// Four consecutive elements of T as floats.
 template <typename T> struct Vec4;
 template <> struct Vec4<uint16_t> {
     static __device__ __forceinline__ void ld(const uint16_t *p, float (&x)[4]) {
@@ -304,21 +304,61 @@ template <> struct Vec4<float> {
     }
 };
 
-// INT8 caches: a KV head's D / 8 lanes reduce the absmax of its D (smoothed) key or value
-// elements with xor shuffles and each lane stores its quantized elements as 32-bit words;
-// the arithmetic is quantize_store's element by element (bit-identical).
-template <typename T, bool NORM, bool INT8, int D>
-__global__ void __launch_bounds__(256) attention_inputs_v_kernel(
+// E consecutive elements of T, loaded, stored, or unpacked from 16 bytes.
+template <typename T, int E> struct VecE;
+template <> struct VecE<float, 4> : Vec4<float> {
+    static __device__ __forceinline__ void unpack(uint4 w, float (&x)[4]) {
+        x[0] = __uint_as_float(w.x);
+        x[1] = __uint_as_float(w.y);
+        x[2] = __uint_as_float(w.z);
+        x[3] = __uint_as_float(w.w);
+    }
+};
+template <> struct VecE<uint16_t, 4> : Vec4<uint16_t> {};
+template <> struct VecE<uint16_t, 8> {
+    static __device__ __forceinline__ void ld(const uint16_t *p, float (&x)[8]) {
+        unpack(*reinterpret_cast<const uint4 *>(p), x);
+    }
+    static __device__ __forceinline__ void unpack(uint4 w, float (&x)[8]) {
+        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            x[2 * e] = __uint_as_float(ws[e] << 16);
+            x[2 * e + 1] = __uint_as_float(ws[e] & 0xffff0000u);
+        }
+    }
+    static __device__ __forceinline__ void st(uint16_t *p, const float (&x)[8]) {
+        *reinterpret_cast<uint4 *>(p) = make_uint4(pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]),
+                                                   pack_bf16x2(x[4], x[5]), pack_bf16x2(x[6], x[7]));
+    }
+};
+
+// The fused kernel for head_dim 128 or 64. A lane owns NE consecutive elements of each half of
+// its head (NE u .. and D/2 + NE u ..), D / (2 NE) lanes per head. A work-group holds heads of
+// one token, so its position, slot and rotary row are uniform.
+// Bound: HBM for prompts (8192 tokens of 32 / 8 heads with the q/k norm: 202 MB in 43.3 us, 4.7
+// TB/s, where a large copy reaches 4.9), the launch and three dependent round trips
+// (arguments, position, rotary row) for few tokens (one: 2.7 us). Value rows stay in two
+// named registers: as an array the compiler kept Float32 ones in LDS (512 tokens of 16 / 8
+// heads 18.6 -> 4.7 us); slots divide in 32 bits.
+// The norm's sum of squares is combined in the one-wave kernel's butterfly order: that
+// kernel's lane i holds a_i^2 + b_i^2 and adds across i ^ 32, 16, 8, 4, 2, 1; here i = NE u + e,
+// so the first steps cross lanes (u ^ 32 / NE, ...) and the last log2(NE) stay in the lane.
+// INT8 caches: a KV head's lanes reduce the absmax of its D (smoothed) key or value elements
+// with xor shuffles; the arithmetic is quantize_store's element by element (bit-identical).
+template <typename T, bool NORM, bool INT8, int D, int NE>
+__global__ void __launch_bounds__(512) attention_inputs_v_kernel(
     T *__restrict__ q_out, T *__restrict__ kp, T *__restrict__ vp, int8_t *__restrict__ lq,
     float *__restrict__ ls, const float *__restrict__ smooth, const T *__restrict__ qkv,
     const T *__restrict__ q_norm, const T *__restrict__ k_norm, const T *__restrict__ cos_sin,
     int table_len, const int32_t *__restrict__ positions, const int32_t *__restrict__ slots,
     int nq, int nkv, int P, int pages, float eps) {
-    constexpr int HALF = D / 2, LPH = D / 8, HPW = 256 / LPH;   // lanes, heads per work-group
+    constexpr int HALF = D / 2, LPH = HALF / NE;   // lanes per head
+    constexpr int VC = D * (int)sizeof(T) / 16 / LPH;   // 16-byte chunks of a value row per lane: u, u + LPH
     using E = Elt<T>;
-    using V = Vec4<T>;
-    const int t = blockIdx.x, j = blockIdx.y * HPW + threadIdx.x / LPH, u = threadIdx.x % LPH;
-    if (j >= nq + nkv) return;   // a whole 16-lane group
+    using V = VecE<T, NE>;
+    const int t = blockIdx.x, j = (blockIdx.y * blockDim.x + threadIdx.x) / LPH, u = threadIdx.x % LPH;
+    if (j >= nq + nkv) return;   // a whole lane group
     const bool is_q = j < nq;
     const int h = j - nq;
     // Every load that does not depend on the position goes out first (token t < n and head
@@ -327,99 +367,91 @@ __global__ void __launch_bounds__(256) attention_inputs_v_kernel(
     const int pos = positions[t];
     const int32_t slot = slots[t];
     const size_t col = ((size_t)t * (nq + 2 * nkv) + j) * D;
-    float a[4], b[4];
-    V::ld(qkv + col + 4 * u, a);
-    V::ld(qkv + col + HALF + 4 * u, b);
-    constexpr int VCH = D * (int)sizeof(T) / 16;   // 16-byte chunks of a value row
-    uint4 vrow[VCH / LPH];
+    float a[NE], b[NE];
+    V::ld(qkv + col + NE * u, a);
+    V::ld(qkv + col + HALF + NE * u, b);
+    uint4 v0 = make_uint4(0, 0, 0, 0), v1 = v0;
     if (!is_q) {
         const uint4 *vs = reinterpret_cast<const uint4 *>(qkv + ((size_t)t * (nq + 2 * nkv) + nq + nkv + h) * D);
-#pragma unroll
-        for (int c = 0; c < VCH / LPH; c++) vrow[c] = vs[u + LPH * c];
+        v0 = vs[u];
+        if (VC == 2) v1 = vs[u + LPH];
     }
-    float w1[4], w2[4];
+    float w1[NE], w2[NE];
     if (NORM) {
         const T *wn = is_q ? q_norm : k_norm;
-        V::ld(wn + 4 * u, w1);
-        V::ld(wn + HALF + 4 * u, w2);
+        V::ld(wn + NE * u, w1);
+        V::ld(wn + HALF + NE * u, w2);
     }
     if (pos < 0 || pos >= table_len) return;
+    const T *cs = cos_sin + (size_t)pos * 2 * D;
+    float c1[NE], c2[NE], s1[NE], s2[NE], y1[NE], y2[NE];
+    V::ld(cs + NE * u, c1);
+    V::ld(cs + HALF + NE * u, c2);
+    V::ld(cs + D + NE * u, s1);
+    V::ld(cs + D + HALF + NE * u, s2);
     long long row = 0;
     if (!is_q) {
         row = slot_row(slot, h, P, nkv, pages);
         if (row < 0) return;
     }
     if (NORM) {
-        float pp[4];
+        float pp[NE];
 #pragma unroll
-        for (int e = 0; e < 4; e++) pp[e] = a[e] * a[e] + b[e] * b[e];
+        for (int e = 0; e < NE; e++) pp[e] = a[e] * a[e] + b[e] * b[e];
 #pragma unroll
         for (int o = LPH / 2; o > 0; o >>= 1)
 #pragma unroll
-            for (int e = 0; e < 4; e++) pp[e] = pp[e] + __shfl_xor(pp[e], o);
-        const float p02 = pp[0] + pp[2], p13 = pp[1] + pp[3];
-        const float ss = p02 + p13;
-        const float inv_rms = __frcp_rn(__fsqrt_rn(__fadd_rn(__fdiv_rn(ss, (float)D), eps)));
+            for (int e = 0; e < NE; e++) pp[e] = pp[e] + __shfl_xor(pp[e], o);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
+        for (int o = NE / 2; o > 0; o >>= 1)
+#pragma unroll
+            for (int e = 0; e < o; e++) pp[e] = pp[e] + pp[e + o];
+        const float inv_rms = __frcp_rn(__fsqrt_rn(__fadd_rn(__fdiv_rn(pp[0], (float)D), eps)));
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
             a[e] = E::rnd(E::rnd(a[e] * inv_rms) * w1[e]);
             b[e] = E::rnd(E::rnd(b[e] * inv_rms) * w2[e]);
         }
     }
-    const T *cs = cos_sin + (size_t)pos * 2 * D;
-    float c1[4], c2[4], s1[4], s2[4], y1[4], y2[4];
-    V::ld(cs + 4 * u, c1);
-    V::ld(cs + HALF + 4 * u, c2);
-    V::ld(cs + D + 4 * u, s1);
-    V::ld(cs + D + HALF + 4 * u, s2);
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
+    for (int e = 0; e < NE; e++) {
         y1[e] = E::rnd(E::rnd(a[e] * c1[e]) + E::rnd(-b[e] * s1[e]));
         y2[e] = E::rnd(E::rnd(b[e] * c2[e]) + E::rnd(a[e] * s2[e]));
     }
     if (!INT8 || is_q) {
         T *dst = is_q ? q_out + ((size_t)t * nq + j) * D : kp + (size_t)row * D;
-        V::st(dst + 4 * u, y1);
-        V::st(dst + HALF + 4 * u, y2);
+        V::st(dst + NE * u, y1);
+        V::st(dst + HALF + NE * u, y2);
         if (is_q) return;
     }
     if constexpr (!INT8) {
-        // the value row (loaded above): a bit copy in 16-byte chunks over the head's lanes
+        // the value row (loaded above): a bit copy
         uint4 *vd = reinterpret_cast<uint4 *>(vp + (size_t)row * D);
-#pragma unroll
-        for (int c = 0; c < VCH / LPH; c++) vd[u + LPH * c] = vrow[c];
+        vd[u] = v0;
+        if (VC == 2) vd[u + LPH] = v1;
     } else {
         const size_t half_q = (size_t)pages * nkv * P * D, half_s = (size_t)pages * nkv * P;
-        // keys: the rotated elements 4u + e and 64 + 4u + e divided by their smoothing
-        float x[8];
+        // keys: the rotated elements divided by their smoothing; values as they are
+        float x[2 * NE];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            x[e] = __fdiv_rn(y1[e], smooth[4 * u + e]);
-            x[4 + e] = __fdiv_rn(y2[e], smooth[HALF + 4 * u + e]);
+        for (int e = 0; e < NE; e++) {
+            x[e] = __fdiv_rn(y1[e], smooth[NE * u + e]);
+            x[NE + e] = __fdiv_rn(y2[e], smooth[HALF + NE * u + e]);
         }
-        quantize_group<LPH>(x, lq + (size_t)row * D, 4 * u, HALF + 4 * u, ls + row, u);
-        // values: this lane's 16-byte chunks of the row, elements in order
-        float v[8];
-        if constexpr (sizeof(T) == 2) {
-            // chunk u = elements 8u .. 8u + 7
-            const uint4 w = vrow[0];
-            const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+        quantize_group<LPH>(x, lq + (size_t)row * D, NE * u, HALF + NE * u, ls + row, u);
+        if constexpr (VC == 2) {
+            float lo[NE], hi[NE];   // chunks u, u + LPH: elements NE u .. and HALF + NE u ..
+            V::unpack(v0, lo);
+            V::unpack(v1, hi);
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                v[2 * e] = __uint_as_float(ws[e] << 16);
-                v[2 * e + 1] = __uint_as_float(ws[e] & 0xffff0000u);
+            for (int e = 0; e < NE; e++) {
+                x[e] = lo[e];
+                x[NE + e] = hi[e];
             }
-            quantize_group<LPH>(v, lq + half_q + (size_t)row * D, 8 * u, 8 * u + 4, ls + half_s + row, u);
+            quantize_group<LPH>(x, lq + half_q + (size_t)row * D, NE * u, HALF + NE * u, ls + half_s + row, u);
         } else {
-            // chunks u and u + LPH = elements 4u .. 4u + 3 and HALF + 4u .. HALF + 4u + 3
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                v[4 * c] = __uint_as_float(vrow[c].x);
-                v[4 * c + 1] = __uint_as_float(vrow[c].y);
-                v[4 * c + 2] = __uint_as_float(vrow[c].z);
-                v[4 * c + 3] = __uint_as_float(vrow[c].w);
-            }
-            quantize_group<LPH>(v, lq + half_q + (size_t)row * D, 4 * u, HALF + 4 * u, ls + half_s + row, u);
+            VecE<uint16_t, 8>::unpack(v0, x);   // chunk u: elements 8 u ..
+            quantize_group<LPH>(x, lq + half_q + (size_t)row * D, 8 * u, 8 * u + 4, ls + half_s + row, u);
         }
     }
 }
@@ -628,14 +660,30 @@ static void launch_inputs(void *q_out, const ti_kv_cache *c, const void *qkv, co
                           const int32_t *positions, const int32_t *slots, int n, int nq,
                           float eps, hipStream_t s) {
     if (c->head_dim == 128 || c->head_dim == 64) {
-        const int hpw = 2048 / c->head_dim;   // heads per 256-thread work-group
-        dim3 grid(n, (nq + c->kv_heads + hpw - 1) / hpw);
-#define TI_INPUTS_V(DD)                                                                            \
-    attention_inputs_v_kernel<T, NORM, INT8, DD><<<grid, 256, 0, s>>>(                             \
+        // Dense bf16 prompts: eight elements per half and lane (16-byte accesses, half the waves;
+        // 8192 tokens 46.7 -> 43.3 us, 512 5.5 -> 5.0). Few tokens: four, since a lane's chain of
+        // shuffles and roundings shows (64 tokens 3.1 against 3.7 us); INT8 too, whose
+        // quantization divides element by element (1500 tokens 12.3 against 13.4), and D = 128
+        // tokens that would leave half a wave idle (36 heads, 2048 tokens: 11.5 against 11.9).
+        const int heads = nq + c->kv_heads;
+        const bool wide = sizeof(T) == 2 && !INT8 && n >= 256 && (c->head_dim == 64 || heads % 8 == 0);
+        // whole heads in work-groups of at most 512 threads, as few as hold a token's heads (few
+        // tokens: 128, so a token spreads over more CUs: 2.75 -> 2.7 us for one)
+        const int lanes = heads * c->head_dim / (wide ? 16 : 8), most = n >= 256 ? 512 : 128;
+        const int parts = (lanes + most - 1) / most, threads = ((lanes + parts - 1) / parts + 63) / 64 * 64;
+        const dim3 grid(n, (lanes + threads - 1) / threads);
+#define TI_INPUTS_V(DD, NE)                                                                        \
+    attention_inputs_v_kernel<T, NORM, INT8, DD, NE><<<grid, threads, 0, s>>>(                     \
         (T *)q_out, (T *)c->k_pages, (T *)c->v_pages, c->layer_q, c->layer_scale, c->smooth,        \
         (const T *)qkv, (const T *)q_norm, (const T *)k_norm, (const T *)cos_sin, table_len,        \
         positions, slots, nq, c->kv_heads, c->page_size, c->num_pages, eps);
-        if (c->head_dim == 128) { TI_INPUTS_V(128) } else { TI_INPUTS_V(64) }
+        if constexpr (sizeof(T) == 2 && !INT8) {
+            if (wide) {
+                if (c->head_dim == 128) { TI_INPUTS_V(128, 8) } else { TI_INPUTS_V(64, 8) }
+                return;
+            }
+        }
+        if (c->head_dim == 128) { TI_INPUTS_V(128, 4) } else { TI_INPUTS_V(64, 4) }
 #undef TI_INPUTS_V
         return;
     }
