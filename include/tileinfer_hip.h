@@ -54,7 +54,8 @@ typedef enum { TI_KV_DENSE = 0, TI_KV_INT8 = 1 } ti_kv_kind;
  *   PREFILL_DIRECT    four-wave kernel, direct global -> LDS tile loads (bf16 dense cache,
  *                     head_dim 128, pages of 2^k >= 16 tokens; otherwise staged)
  *   PREFILL_PINGPONG  eight-wave ping-pong kernel, 256 packed rows per work-group (bf16 dense
- *                     cache, head_dim 128, pages of 2^k >= 16 tokens)
+ *                     cache, head_dim 128, pages of 2^k >= 16 tokens, 256 % (q_heads /
+ *                     kv_heads) == 0)
  *   PREFILL_PAIRED    four-wave kernel with direct loads whose work-groups each take a
  *                     heavy and a light 32-row q-tile of a causal step (direct-load shapes,
  *                     32 % (q_heads / kv_heads) == 0, the shapes' unsplit two-wave plan)

@@ -1214,9 +1214,11 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     const long long pairs = (long long)c->kv_heads * a->num_seqs;
     const long long key_tiles = ((long long)a->block_table_stride * c->page_size + 31) / 32;
     // PAIRED16 pins the 16-row kernel where it is not beaten: launches that the library gives
-    // to the ping-pong kernel on a dense cache fall back to that pick.
+    // to the ping-pong kernel on a dense cache fall back to that pick. (Those whose pairs of
+    // q-tiles exceed a grid keep the paired plan, which is refused.)
     int path = a->path;
-    if (path == TI_PATH_PREFILL_PAIRED16 && c->kind == TI_KV_DENSE && ti_pick_prefill_pp(a, c, TI_PATH_AUTO))
+    if (path == TI_PATH_PREFILL_PAIRED16 && c->kind == TI_KV_DENSE && a->causal && 32 % G == 0 &&
+        ((a->max_query_len + 32LL / G - 1) / (32 / G) + 1) / 2 <= 65535 && ti_pick_prefill_pp(a, c, TI_PATH_AUTO))
         path = TI_PATH_AUTO;
     const bool auto_path = path == TI_PATH_PREFILL || path == TI_PATH_AUTO;
     pl.pp = ti_pick_prefill_pp(a, c, path);

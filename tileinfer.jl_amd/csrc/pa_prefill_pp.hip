@@ -636,9 +636,11 @@ int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int pat
         2ull * c->kv_heads * P * D > 0xffffffffull)
         return TI_PP_NONE;
     const bool dense = c->kind == TI_KV_DENSE, dense128 = dense && D == 128;
-    if (path == TI_PATH_PREFILL_PINGPONG && dense128) return TI_PP_SHARED;
+    if (path == TI_PATH_PREFILL_PINGPONG && dense128 && 256 % G == 0) return TI_PP_SHARED;
     if (path != TI_PATH_AUTO && path != TI_PATH_PREFILL) return TI_PP_NONE;
     const long long TQ = 128 / G, T = (a->max_query_len + TQ - 1) / TQ, W = T * c->kv_heads * a->num_seqs;
+    // grids hold 65535 q-tiles: 256-row ones where those have been taken, none where not
+    if (T > 65535) return dense128 && 256 % G == 0 ? TI_PP_SHARED : TI_PP_NONE;
     if (T <= 2) return W >= 512 ? TI_PP_SOLO : (D == 128 && W >= (dense ? 129 : 256) ? TI_PP_KSPLIT : TI_PP_NONE);
     const int first = dense ? (128 % G == 0 ? 129 : 160) : (a->num_seqs > 1 ? 160 : D == 64 ? 256 : 257);
     if (W < first) return TI_PP_NONE;
