@@ -1,4 +1,5 @@
-"""Build libtileinfer_hip.so for gfx950 from csrc/*.hip with hipcc (no GPU needed).
+"""Build libtileinfer_hip.so for gfx950 from csrc/*.hip with hipcc, and the Python package's
+native call path _calls.so from csrc/py_calls.cpp with g++ (no GPU needed).
 
     python tileinfer.jl_amd/build.py
 
@@ -18,6 +19,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 OUT = os.path.join(PKG, "tileinfer_hip", "libtileinfer_hip.so")
+CALLS = os.path.join(PKG, "tileinfer_hip", "_calls.so")
 BUILD = os.path.join(ROOT, "_build")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -45,15 +47,38 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_calls() -> str:
+    """_calls.so: a CPython module against torch's headers (host code only)."""
+    import sysconfig
+
+    import torch
+
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I", os.path.join(ROOT, "include"), "-isystem", inc,
+           "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", sysconfig.get_paths()["include"],
+           "-isystem", "/opt/rocm/include", os.path.join(CSRC, "py_calls.cpp"), "-o", CALLS, "-L", lib,
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{lib}"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        sys.stderr.write(r.stdout + r.stderr)
+        raise RuntimeError("g++ failed on py_calls.cpp")
+    return CALLS
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(BUILD, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        calls = ex.submit(_build_calls)
         objs = list(ex.map(_compile, srcs))
+        calls.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", OUT, *objs]
     subprocess.run(cmd, check=True)
     if verbose:
-        print("built", OUT)
+        print("built", OUT, CALLS)
     return OUT
 
 

@@ -76,8 +76,33 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     L.ti_attention_inputs.restype = i32
     L.ti_attention_inputs.argtypes = [i32, vp, P(KVCache), vp, vp, vp, vp, i32, vp, vp, i32, i32,
                                       ctypes.c_float, vp]
+    _bind_calls(L)
     _lib = L
     return L
+
+
+calls = None
+
+
+def _bind_calls(L: ctypes.CDLL) -> None:
+    """Point the native call path (_calls.so) at the loaded library's entry points."""
+    global calls
+    from .kv import Int8Pages
+    try:
+        from . import _calls
+    except ImportError as e:
+        raise RuntimeError("tileinfer_hip/_calls.so is missing or does not fit this torch: "
+                           "build it with `python tileinfer.jl_amd/build.py`") from e
+    _calls.bind(Int8Pages, *(ctypes.cast(f, ctypes.c_void_p).value for f in
+                             (L.ti_attention, L.ti_attention_inputs, L.ti_store_kv, L.ti_rope, L.ti_rmsnorm)))
+    calls = _calls
+
+
+def native():
+    """The native call path; loads the library on first use."""
+    if calls is None:
+        load()
+    return calls
 
 
 class TileInferError(RuntimeError):

@@ -24,6 +24,14 @@ from .kv import Int8Pages, layer_arrays
 from .rope import RotaryTable
 
 
+def _done(status: int) -> bool:
+    """Whether the native call path made a call (raising what it reported): it leaves
+    arguments that are not plain ones (-1) to the checks below."""
+    if status > 0:
+        check(status)
+    return status == 0
+
+
 class HipBackend:
     """Selects the MI355X kernels, as TileBackend selects the cuTile ones
     (src/ops/interface.jl:15-21)."""
@@ -154,6 +162,9 @@ def paged_attention_(be: HipBackend, out, workspace, q, k_pages, v_pages, block_
                      max_query_len: Optional[int] = None, path: int = _lib.TI_PATH_AUTO):
     """Batched attention_: sequence b owns tokens [qsl[b], qsl[b+1]) of q (or equal
     shares when query_start_loc is None) and block table row block_tables[b]."""
+    if _done(_lib.native().attention(out, workspace, q, k_pages, v_pages, block_tables, positions, scale, causal,
+                                     query_start_loc, max_query_len, path, False)):
+        return out
     bts = block_tables if block_tables.dim() == 2 else block_tables.view(1, -1)
     B = bts.shape[0]
     _dev(out, q, bts, positions, query_start_loc, workspace)
@@ -181,6 +192,9 @@ def attention_(be: HipBackend, out, workspace, q, k_pages, v_pages, block_table,
                scale: float, causal: bool = True, path: int = _lib.TI_PATH_AUTO):
     """attention!(::TileBackend, out, workspace, q, k_pages, v_pages, block_table,
     positions, scale; causal) (src/ops/tile/attention.jl:359-366) for one sequence."""
+    if _done(_lib.native().attention(out, workspace, q, k_pages, v_pages, block_table, positions, scale, causal,
+                                     None, None, path, True)):
+        return out
     return paged_attention_(be, out, workspace, q, k_pages, v_pages, block_table.view(1, -1),
                             positions, scale, causal, path=path)
 
@@ -196,6 +210,8 @@ def attention(be: HipBackend, q, k_pages, v_pages, block_table, positions, scale
 def store_kv_(be: HipBackend, k_pages, v_pages, k, v, slots):
     """store_kv!(::TileBackend, k_pages, v_pages, k, v, slots)
     (src/ops/tile/elementwise.jl:133-140, :180-188)."""
+    if _done(_lib.native().store_kv(k_pages, v_pages, k, v, slots)):
+        return
     _dev(k, v, slots)
     _i32(slots, "slots")
     if k.shape != v.shape or k.dtype != v.dtype or k.dim() != 3:
@@ -210,6 +226,8 @@ def store_kv_(be: HipBackend, k_pages, v_pages, k, v, slots):
 def rmsnorm_(be: HipBackend, y, x, w, eps: float):
     """rmsnorm!(::TileBackend, y, x, w, eps) (src/ops/tile/norm.jl:31-38): every row of the
     last dimension of x normalized as rnd(rnd(x inv_rms) w). y may be x."""
+    if _done(_lib.native().rmsnorm(y, x, w, eps)):
+        return y
     _dev(y, x, w)
     if y.shape != x.shape or y.dtype != x.dtype or w.dtype != x.dtype or w.dim() != 1 \
             or w.shape[0] != x.shape[-1] or not (x.is_contiguous() and y.is_contiguous()):
@@ -227,6 +245,8 @@ def rmsnorm(be: HipBackend, x, w, eps: float):
 def rope_(be: HipBackend, y, x, cos, sin, positions):
     """rope!(::TileBackend, y, x, cos, sin, positions) (src/ops/tile/elementwise.jl:29-36).
     cos/sin: [max_len][D]."""
+    if _done(_lib.native().rope(y, x, cos, sin, positions)):
+        return y
     _dev(y, x, cos, sin, positions)
     _i32(positions, "positions")
     if x.dim() != 3 or y.shape != x.shape or y.dtype != x.dtype or cos.dtype != x.dtype \
@@ -249,6 +269,8 @@ def attention_inputs_(be: HipBackend, q, k_pages, v_pages, qkv, q_norm, k_norm,
     """attention_inputs!(::TileBackend, q, k_pages, v_pages, qkv, q_norm, k_norm, table,
     positions, slots, eps) (src/ops/tile/fused.jl:94-130): optional q/k RMSNorm, RoPE,
     queries into q, keys and values into the cache; returns q."""
+    if _done(_lib.native().attention_inputs(q, k_pages, v_pages, qkv, q_norm, k_norm, table, positions, slots, eps)):
+        return q
     _dev(q, qkv, q_norm, k_norm, table.cos_sin, positions, slots)
     _i32(positions, "positions")
     _i32(slots, "slots")
