@@ -102,6 +102,17 @@ void launch_decode_d(const DecodeParams &p, int rowb, dim3 grid, hipStream_t s) 
     // 8-wave groups only for up to 32 packed rows (their merge slabs must fit the LDS).
     // 33-64 rows: 4-wave groups of two wave pairs, each pair splitting the rows over the
     // same keys (32 rows per wave keeps the accumulators in VGPRs at 2 waves per SIMD).
+    // INT8 launches of at most one work-group per CU take the joint steps, whose 266 VGPRs leave
+    // one wave per SIMD: Llama-3-8B B = 8 x 32768 94.2 -> 91.7 us, lengths U[1000, 8000] 25.5 ->
+    // 24.3, 4 x U[200, 2000] 11.9 -> 11.5. Larger ones need the second work-group on a CU
+    // (100 sequences of up to 1000: 36.4 against 44.7 us joint; held to 256 VGPRs the joint step
+    // spills, 115.7 us at 8 x 32768). bf16 tiles in pairs gained nothing at head_dim 64 or 128.
+    if constexpr (INT8 && D == 128 && NW == 4) {
+        if (rowb == 1 && (unsigned long long)grid.x * grid.y * grid.z <= 256) {
+            decode_kernel<D, 1, INT8, PG16, NW, 1, true><<<grid, NW * 64, 0, s>>>(p);
+            return;
+        }
+    }
     switch (rowb) {
         case 1: decode_kernel<D, 1, INT8, PG16, NW, 1><<<grid, NW * 64, 0, s>>>(p); break;
         case 2: decode_kernel<D, 2, INT8, PG16, NW, 1><<<grid, NW * 64, 0, s>>>(p); break;

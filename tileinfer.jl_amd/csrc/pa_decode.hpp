@@ -41,6 +41,8 @@
 // w_s = exp2(m_s - max m), o = sum acc_s w_s / sum l_s w_s.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 
 using namespace ti;
@@ -272,7 +274,7 @@ __device__ __forceinline__ void load_tile(TileRegs<D, INT8> &t, const DecodePara
     }
 }
 
-template <int D, int ROWB, bool INT8, bool PG16, int NW, int RS>
+template <int D, int ROWB, bool INT8, bool PG16, int NW, int RS, bool JOINT = false>
 __global__ void __launch_bounds__(NW * 64) decode_kernel(DecodeParams p) {
     constexpr int NKB = D / 32;          // 32-wide head-dim blocks (QK MFMAs per tile)
     constexpr int NDT = D / 16;          // 16-wide head-dim tiles (PV MFMAs per tile)
@@ -280,15 +282,19 @@ __global__ void __launch_bounds__(NW * 64) decode_kernel(DecodeParams p) {
     constexpr int KPL = 16 * CPR / 64;   // keys per lane in the V load (4 for D=128)
     constexpr int MP = ROWB * 16;        // padded rows per wave
     constexpr int NKW = NW / RS;         // waves splitting the keys (RS row slices each)
+    // Tiles loaded per step (TPI: see the loop) and worked on together (JT). JOINT: a whole step
+    // runs its tiles through one softmax, so their score chains overlap and one max decides the
+    // rescale.
+    constexpr int TPI = INT8 ? (ROWB == 1 ? 3 : 2) : 1, JT = JOINT ? TPI : 1;
 
     // Per-wave transposed V tiles during the key loop; afterwards the same LDS holds each
     // wave's (O, m, l) slab for the merge (rows of D + 4 floats, 16-B aligned).
     constexpr int MROW = D + 4;
     constexpr int VROW = vtile_row<D>();
-    constexpr int VT_BYTES = NW * 16 * VROW * 2;
+    constexpr int VT_BYTES = NW * JT * 16 * VROW * 2;
     constexpr int SLAB_BYTES = NW * MP * MROW * 4;
     __shared__ __attribute__((aligned(16))) char smem_raw[VT_BYTES > SLAB_BYTES ? VT_BYTES : SLAB_BYTES];
-    uint16_t (*vt)[16 * VROW] = reinterpret_cast<uint16_t (*)[16 * VROW]>(smem_raw);
+    uint16_t (*vt)[JT * 16 * VROW] = reinterpret_cast<uint16_t (*)[JT * 16 * VROW]>(smem_raw);
     float *mslab = reinterpret_cast<float *>(smem_raw);
 
     const int lane = threadIdx.x & 63;
@@ -401,54 +407,66 @@ __global__ void __launch_bounds__(NW * 64) decode_kernel(DecodeParams p) {
     uint16_t *myvt = vt[w];
     const int vc = lane % CPR, vg = lane / CPR;   // V load: chunk, key group
 
-    auto compute = [&](const TileRegs<D, INT8> &t, int j) {
-        // ---- V rows -> row-major LDS tile (INT8: biased fp16, exact) ----
-        u32x4 vrows[KPL];
+    // NT tiles j .. j + NT - 1: their scores, one softmax over them, their values.
+    auto compute = [&](const TileRegs<D, INT8> *t, int j, auto count) {
+        constexpr int NT = decltype(count)::value;
+        // ---- V rows -> row-major LDS tiles (INT8: biased fp16, exact) ----
+        u32x4 vrows[NT][KPL];
 #pragma unroll
-        for (int e = 0; e < KPL; e++) vrows[e] = INT8 ? i8x8_to_f16b(t.v[e][0], t.v[e][1]) : t.v[e];
-        lds_fence();   // the previous tile's reads of myvt are done before overwriting
+        for (int n = 0; n < NT; n++)
 #pragma unroll
-        for (int e = 0; e < KPL; e++)
-            *reinterpret_cast<u32x4 *>(myvt + (vg * KPL + e) * VROW + vc * 8) = vrows[e];
+            for (int e = 0; e < KPL; e++)
+                vrows[n][e] = INT8 ? i8x8_to_f16b(t[n].v[e][0], t[n].v[e][1]) : t[n].v[e];
+        lds_fence();   // the previous step's reads of myvt are done before overwriting
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int e = 0; e < KPL; e++)
+                *reinterpret_cast<u32x4 *>(myvt + n * 16 * VROW + (vg * KPL + e) * VROW + vc * 8) = vrows[n][e];
         // ---- S^T = K Q^T ----
-        u32x4 kreg[NKB];
+        f32x4 sc[NT][ROWB];
 #pragma unroll
-        for (int i = 0; i < NKB; i++) kreg[i] = INT8 ? i8x8_to_f16b(t.k[i][0], t.k[i][1]) : t.k[i];
-        f32x4 sc[ROWB];
+        for (int n = 0; n < NT; n++) {
+            u32x4 kreg[NKB];
 #pragma unroll
-        for (int rb = 0; rb < ROWB; rb++) {
-            sc[rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < NKB; i++) kreg[i] = INT8 ? i8x8_to_f16b(t[n].k[i][0], t[n].k[i][1]) : t[n].k[i];
 #pragma unroll
-            for (int i = 0; i < NKB; i++) sc[rb] = qk_mfma<INT8>(kreg[i], qreg[rb][i], sc[rb]);
-        }
-        // Scales of this lane's 4 score keys (kg*4 + e), from the lanes that loaded them.
-        float skk[4], svk[4];
-        if (INT8) {
+            for (int rb = 0; rb < ROWB; rb++) {
+                sc[n][rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                skk[e] = __shfl(t.sk, kg * 4 + e);
-                svk[e] = __shfl(t.sv, kg * 4 + e);
+                for (int i = 0; i < NKB; i++) sc[n][rb] = qk_mfma<INT8>(kreg[i], qreg[rb][i], sc[n][rb]);
             }
         }
+        // Scales of this lane's 4 score keys (kg*4 + e) of each tile, from the lanes that loaded them.
+        float skk[NT][4], svk[NT][4];
+        if (INT8) {
+#pragma unroll
+            for (int n = 0; n < NT; n++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    skk[n][e] = __shfl(t[n].sk, kg * 4 + e);
+                    svk[n][e] = __shfl(t[n].sv, kg * 4 + e);
+                }
+        }
         // ---- online softmax + P^T operands ----
-        // Lazy rescaling: m is a reference max that only moves when a tile's max exceeds
+        // Lazy rescaling: m is a reference max that only moves when a step's max exceeds
         // it by more than RESCALE_LOG2 (then p <= 2^RESCALE_LOG2, safe in bf16 and fp32);
         // l and O always use the same reference, so the result is exact. INT8 moves m
         // with every larger max (p <= 1, so p times a value scale stays within fp16).
-        const bool need_mask = j * 16 + 15 > mask_from;
-        s16x4 pop[ROWB];
-        float x[ROWB][4], mt[ROWB];
+        const bool need_mask = (j + NT) * 16 - 1 > mask_from;
+        s16x4 pop[NT][ROWB];
+        float x[ROWB][4 * NT], mt[ROWB];
         bool grow = false;
 #pragma unroll
         for (int rb = 0; rb < ROWB; rb++) {
             mt[rb] = -INFINITY;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                float v = sc[rb][e];
-                if (INT8) v = (v - qcorr[rb]) * skk[e] * qsl[rb];
+            for (int e = 0; e < 4 * NT; e++) {
+                float v = sc[e >> 2][rb][e & 3];
+                if (INT8) v = (v - qcorr[rb]) * skk[e >> 2][e & 3] * qsl[rb];
                 else v *= p.scale_log2;
                 if (need_mask) {
-                    const int kp = j * 16 + kg * 4 + e;
+                    const int kp = (j + (e >> 2)) * 16 + kg * 4 + (e & 3);
                     v = (kp <= qpos[rb] && kp < len) ? v : -INFINITY;
                 }
                 x[rb][e] = v;
@@ -471,35 +489,39 @@ __global__ void __launch_bounds__(NW * 64) decode_kernel(DecodeParams p) {
             }
         }
 #pragma unroll
-        for (int rb = 0; rb < ROWB; rb++) {
-            float ps = 0.0f, pe[4];
+        for (int rb = 0; rb < ROWB; rb++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                pe[e] = fast_exp2(x[rb][e] - m[rb]);
-                ps += pe[e];
-                if (INT8) pe[e] *= svk[e];
+            for (int n = 0; n < NT; n++) {
+                float ps = 0.0f, pe[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    pe[e] = fast_exp2(x[rb][4 * n + e] - m[rb]);
+                    ps += pe[e];
+                    if (INT8) pe[e] *= svk[n][e];
+                }
+                l[rb] += ps;
+                if (INT8) {
+                    const f16x2 h0 = __builtin_convertvector(((f32x2){pe[0], pe[1]}), f16x2);
+                    const f16x2 h1 = __builtin_convertvector(((f32x2){pe[2], pe[3]}), f16x2);
+                    pop[n][rb] = __builtin_bit_cast(s16x4, (u32x2){__builtin_bit_cast(uint32_t, h0),
+                                                                   __builtin_bit_cast(uint32_t, h1)});
+                    // the row's sum of these fp16 probabilities, for the values' bias
+                    const s16x4 ones = __builtin_bit_cast(s16x4, (u32x2){0x3c003c00u, 0x3c003c00u});
+                    psum[rb] = pv_mfma<true>(ones, pop[n][rb], psum[rb]);
+                } else {
+                    pop[n][rb] = __builtin_bit_cast(s16x4, (u32x2){pack_bf16x2(pe[0], pe[1]), pack_bf16x2(pe[2], pe[3])});
+                }
             }
-            l[rb] += ps;
-            if (INT8) {
-                const f16x2 h0 = __builtin_convertvector(((f32x2){pe[0], pe[1]}), f16x2);
-                const f16x2 h1 = __builtin_convertvector(((f32x2){pe[2], pe[3]}), f16x2);
-                pop[rb] = __builtin_bit_cast(s16x4, (u32x2){__builtin_bit_cast(uint32_t, h0),
-                                                            __builtin_bit_cast(uint32_t, h1)});
-                // the row's sum of these fp16 probabilities, for the values' bias
-                const s16x4 ones = __builtin_bit_cast(s16x4, (u32x2){0x3c003c00u, 0x3c003c00u});
-                psum[rb] = pv_mfma<true>(ones, pop[rb], psum[rb]);
-            } else {
-                pop[rb] = __builtin_bit_cast(s16x4, (u32x2){pack_bf16x2(pe[0], pe[1]), pack_bf16x2(pe[2], pe[3])});
-            }
-        }
         // ---- O^T += V^T P^T ----
-        lds_fence();   // this tile's V^T is in LDS
+        lds_fence();   // this step's V^T is in LDS
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) {
-            const s16x4 a = lds_tr16(myvt + (4 * kg + (r16 >> 2)) * VROW + dt * 16 + 4 * (r16 & 3));
+        for (int n = 0; n < NT; n++)
 #pragma unroll
-            for (int rb = 0; rb < ROWB; rb++) o[rb][dt] = pv_mfma<INT8>(a, pop[rb], o[rb][dt]);
-        }
+            for (int dt = 0; dt < NDT; dt++) {
+                const s16x4 a = lds_tr16(myvt + n * 16 * VROW + (4 * kg + (r16 >> 2)) * VROW + dt * 16 + 4 * (r16 & 3));
+#pragma unroll
+                for (int rb = 0; rb < ROWB; rb++) o[rb][dt] = pv_mfma<INT8>(a, pop[n][rb], o[rb][dt]);
+            }
     };
 
     // Two register sets, ping-ponged: the next group of TPI tiles is loading while the
@@ -509,7 +531,6 @@ __global__ void __launch_bounds__(NW * 64) decode_kernel(DecodeParams p) {
     // two for 32-row waves, whose accumulators leave less room. The prefetch is issued
     // unconditionally (past the last tile it re-reads that tile, unused) so the count of
     // loads in flight is static and each wait covers only the tiles in use.
-    constexpr int TPI = INT8 ? (ROWB == 1 ? 3 : 2) : 1;
     constexpr int STRIDE = NKW * TPI;
     TileRegs<D, INT8> ta[TPI], tb[TPI];
     auto ld = [&](TileRegs<D, INT8> (&t)[TPI], int jj) {
@@ -518,9 +539,12 @@ __global__ void __launch_bounds__(NW * 64) decode_kernel(DecodeParams p) {
             load_tile<D, INT8, PG16>(t[e], p, rm, min(jj + e, j1 - 1), r16, kg, vg, vc, half_q, half_s);
     };
     auto run = [&](const TileRegs<D, INT8> (&t)[TPI], int jj) {
+        if constexpr (JT > 1) {
+            if (jj + JT <= j1) return compute(t, jj, std::integral_constant<int, JT>{});
+        }
 #pragma unroll
         for (int e = 0; e < TPI; e++)
-            if (jj + e < j1) compute(t[e], jj + e);
+            if (jj + e < j1) compute(t + e, jj + e, std::integral_constant<int, 1>{});
     };
     int j = j0 + TPI * kw;
     if (j < j1) {
