@@ -38,6 +38,9 @@ CASES = {
     "solo_int8": ("int8", 128, 32, 8, 16, [(0, 700), (333, 650), (0, 0), (12, 32)], True),
     "solo_int8_d64": ("int8", 64, 32, 8, 32, [(0, 700), (333, 650), (1, 1), (12, 32)], True),
     "shared_dense": ("bf16", 128, 32, 8, 16, [(5, 600), (0, 601), (950, 2), (0, 0)], True),
+    # an empty sequence in a step whose first position is 0: no key tile, no page to look up
+    "paired16_empty_first": ("bf16", 128, 32, 8, 16, [(0, 0), (0, 130), (700, 40)], True),
+    "paired16_int8_empty_first": ("int8", 128, 32, 8, 16, [(0, 0), (0, 130), (100, 40)], True),
 }
 
 

@@ -1041,23 +1041,25 @@ __global__ void __launch_bounds__(1024) prefill16_kernel(PrefillParams p) {
     };
 
     auto tile_of = [&](int i) { return grp + NG * i; };
-    const int ft = min(tile_of(0), nkt - 1);
+    // a sequence with no query in the step and no key before it (nkt = 0) looks up tile 0, which
+    // nothing uses
+    const int last_tile = max(nkt - 1, 0), ft = min(tile_of(0), last_tile);
     TilePages pn = ft == grp ? spec : raw_pages(p, bt, ft);
     // A step issues the next tile's loads first and looks up the page ids of the tile after
     // at its end (next_pages), so the scalar loads' wait falls on the step's closing barrier
     // instead of on its LDS reads (both are counted by lgkmcnt).
     auto issue = [&](int i, int buf) {
-        if (i < steps) dl_load(min(tile_of(i), nkt - 1), buf, pn);
+        if (i < steps) dl_load(min(tile_of(i), last_tile), buf, pn);
     };
     auto next_pages = [&](int i) {
-        if (i < steps) pn = raw_pages(p, bt, min(tile_of(i), nkt - 1));
+        if (i < steps) pn = raw_pages(p, bt, min(tile_of(i), last_tile));
     };
     if constexpr (!INT8) {
         if (!first_full) issue(0, 0);
         next_pages(1);
     } else {
-        i8_load(min(tile_of(0), nkt - 1), pn);
-        pn = raw_pages(p, bt, min(tile_of(1), nkt - 1));
+        i8_load(min(tile_of(0), last_tile), pn);
+        pn = raw_pages(p, bt, min(tile_of(1), last_tile));
         i8_store(0);
     }
     wait_direct_loads();   // the queries' direct loads (and tile 0's)
