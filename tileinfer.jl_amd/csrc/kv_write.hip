@@ -661,15 +661,21 @@ static void launch_inputs(void *q_out, const ti_kv_cache *c, const void *qkv, co
                           float eps, hipStream_t s) {
     if (c->head_dim == 128 || c->head_dim == 64) {
         // Dense bf16 prompts: eight elements per half and lane (16-byte accesses, half the waves;
-        // 8192 tokens 46.7 -> 43.3 us, 512 5.5 -> 5.0). Few tokens: four, since a lane's chain of
-        // shuffles and roundings shows (64 tokens 3.1 against 3.7 us); INT8 too, whose
-        // quantization divides element by element (1500 tokens 12.3 against 13.4), and D = 128
-        // tokens that would leave half a wave idle (36 heads, 2048 tokens: 11.5 against 11.9).
+        // 8192 tokens 46.7 -> 43.3 us, 512 5.5 -> 5.0) where that leaves five waves to a CU. With
+        // fewer a lane's chain of shuffles and roundings shows (64 tokens 3.1 against 3.7 us, 300
+        // of 16 / 8 heads 4.0 against 4.2). INT8 takes four, since its quantization divides element
+        // by element (1500 tokens 12.3 against 13.4), and so do D = 128 tokens that would leave
+        // half a wave idle (36 heads, 2048 tokens: 11.5 against 11.9).
         const int heads = nq + c->kv_heads;
-        const bool wide = sizeof(T) == 2 && !INT8 && n >= 256 && (c->head_dim == 64 || heads % 8 == 0);
-        // whole heads in work-groups of at most 512 threads, as few as hold a token's heads (few
-        // tokens: 128, so a token spreads over more CUs: 2.75 -> 2.7 us for one)
-        const int lanes = heads * c->head_dim / (wide ? 16 : 8), most = n >= 256 ? 512 : 128;
+        const bool wide = sizeof(T) == 2 && !INT8 && (long long)n * heads * c->head_dim >= 5ll * 256 * 1024 &&
+                          (c->head_dim == 64 || heads % 8 == 0);
+        // Work-groups of one wave as long as all waves fit the chip at once (32 per CU), so that no
+        // CU gets a whole token more than another (300 tokens 5.2 -> 4.7 us, 1500 13.1 -> 11.8, INT8 700 8.5 -> 7.7, of
+        // 16 / 8 Float32 heads 300 4.6 -> 4.2); beyond, whole tokens in up to 512 threads (4000
+        // tokens of 16 / 8 heads 17.0 against 17.7, Float32 27.2 against 30.4). Up to 255 tokens
+        // 128 threads (one token 2.75 against 2.85, 130 tokens 3.4 against 3.5).
+        const int lanes = heads * c->head_dim / (wide ? 16 : 8);
+        const int most = n < 256 ? 128 : (long long)n * lanes < 64ll * 32 * 256 ? 64 : 512;
         const int parts = (lanes + most - 1) / most, threads = ((lanes + parts - 1) / parts + 63) / 64 * 64;
         const dim3 grid(n, (lanes + threads - 1) / threads);
 #define TI_INPUTS_V(DD, NE)                                                                        \
