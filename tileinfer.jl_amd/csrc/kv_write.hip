@@ -670,10 +670,11 @@ static void launch_inputs(void *q_out, const ti_kv_cache *c, const void *qkv, co
         const bool wide = sizeof(T) == 2 && !INT8 && (long long)n * heads * c->head_dim >= 5ll * 256 * 1024 &&
                           (c->head_dim == 64 || heads % 8 == 0);
         // Work-groups of one wave as long as all waves fit the chip at once (32 per CU), so that no
-        // CU gets a whole token more than another (300 tokens 5.2 -> 4.7 us, 1500 13.1 -> 11.8, INT8 700 8.5 -> 7.7, of
-        // 16 / 8 Float32 heads 300 4.6 -> 4.2); beyond, whole tokens in up to 512 threads (4000
-        // tokens of 16 / 8 heads 17.0 against 17.7, Float32 27.2 against 30.4). Up to 255 tokens
-        // 128 threads (one token 2.75 against 2.85, 130 tokens 3.4 against 3.5).
+        // CU gets a whole token more than another (300 tokens 5.2 -> 4.7 us, 1500 13.1 -> 11.8,
+        // INT8 700 8.5 -> 7.7, of 16 / 8 Float32 heads 300 4.6 -> 4.2); beyond, whole tokens in up
+        // to 512 threads (4000 tokens of 16 / 8 heads 17.0 against 17.7, Float32 27.2 against
+        // 30.4). Up to 255 tokens 128 threads (one token 2.75 against 2.85, 130 tokens 3.4
+        // against 3.5).
         const int lanes = heads * c->head_dim / (wide ? 16 : 8);
         const int most = n < 256 ? 128 : (long long)n * lanes < 64ll * 32 * 256 ? 64 : 512;
         const int parts = (lanes + most - 1) / most, threads = ((lanes + parts - 1) / parts + 63) / 64 * 64;
