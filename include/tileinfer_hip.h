@@ -60,8 +60,8 @@ typedef enum { TI_KV_DENSE = 0, TI_KV_INT8 = 1 } ti_kv_kind;
  *                     heavy and a light 32-row q-tile of a causal step (direct-load shapes,
  *                     32 % (q_heads / kv_heads) == 0, the shapes' unsplit two-wave plan)
  *   PREFILL_PAIRED16  the same paired work-groups on sixteen waves of 16 rows each (four
- *                     per SIMD; on a dense cache only launches of up to 256 pairs, where no
- *                     form of the ping-pong kernel is faster, the default there) */
+ *                     per SIMD; the default where the paired plan applies and no form of the
+ *                     ping-pong kernel is taken) */
 typedef enum {
     TI_PATH_AUTO = 0,
     TI_PATH_DECODE = 1,

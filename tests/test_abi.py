@@ -162,6 +162,17 @@ def test_paired_prefill_grid_counts_pairs():
             assert L.ti_attention(ctypes.byref(a), ctypes.byref(c), None) == want
 
 
+def test_pinned_prefill_variants_keep_their_plan():
+    """A pinned path is not handed to another kernel: 24 sequences of 16 tokens (G = 4) split
+    their keys on the four-wave plan, which the paired variants fall back to where keys split,
+    so every path pinned to that family asks for the split partials, whatever AUTO takes."""
+    want = 24 * 8 * 2 * 64 * 130 * 4       # 2 splits of 64 packed rows of D + 2 floats
+    for path in (_lib.TI_PATH_PREFILL_STAGED, _lib.TI_PATH_PREFILL_DIRECT, _lib.TI_PATH_PREFILL_PAIRED,
+                 _lib.TI_PATH_PREFILL_PAIRED16):
+        a = _args(num_seqs=24, max_query_len=16, total_tokens=24 * 16, block_table_stride=512, path=path)
+        assert ws(a, _cache()) == (_lib.TI_OK, want), path
+
+
 def test_store_rope_inputs_validation():
     L = ti.load_library()
     c = _cache()

@@ -1226,15 +1226,8 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     const int G = a->q_heads / c->kv_heads;
     const long long pairs = (long long)c->kv_heads * a->num_seqs;
     const long long key_tiles = ((long long)a->block_table_stride * c->page_size + 31) / 32;
-    // PAIRED16 pins the 16-row kernel where it is not beaten: launches that the library gives
-    // to the ping-pong kernel on a dense cache fall back to that pick. (Those whose pairs of
-    // q-tiles exceed a grid keep the paired plan, which is refused.)
-    int path = a->path;
-    if (path == TI_PATH_PREFILL_PAIRED16 && c->kind == TI_KV_DENSE && a->causal && 32 % G == 0 &&
-        ((a->max_query_len + 32LL / G - 1) / (32 / G) + 1) / 2 <= 65535 && ti_pick_prefill_pp(a, c, TI_PATH_AUTO))
-        path = TI_PATH_AUTO;
-    const bool auto_path = path == TI_PATH_PREFILL || path == TI_PATH_AUTO;
-    pl.pp = ti_pick_prefill_pp(a, c, path);
+    const bool auto_path = a->path == TI_PATH_PREFILL || a->path == TI_PATH_AUTO;
+    pl.pp = ti_pick_prefill_pp(a, c, a->path);
     pl.dl = 0;
     pl.pair = 0;
     pl.r16 = 0;
@@ -1273,9 +1266,9 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     // (1024-3072 tokens) no change, so those keep the register-staged loads.
     const bool dl_ok = c->kind == TI_KV_DENSE && a->dtype == TI_BF16 && c->head_dim == 128 &&
                        c->page_size >= 16 && (c->page_size & (c->page_size - 1)) == 0;
-    pl.dl = dl_ok && (path == TI_PATH_PREFILL_DIRECT || path == TI_PATH_PREFILL_PAIRED ||
-                      path == TI_PATH_PREFILL_PAIRED16 ||
-                      (path != TI_PATH_PREFILL_STAGED && pl.wpg == 2));
+    pl.dl = dl_ok && (a->path == TI_PATH_PREFILL_DIRECT || a->path == TI_PATH_PREFILL_PAIRED ||
+                      a->path == TI_PATH_PREFILL_PAIRED16 ||
+                      (a->path != TI_PATH_PREFILL_STAGED && pl.wpg == 2));
     // Paired q-tiles (a heavy and a light 32-row q-tile per work-group, equal causal work
     // per work-group) for causal steps without key splits on the direct-load shapes; G
     // must divide 32 (whole positions per 32-row q-tile). On 16-row waves
@@ -1292,9 +1285,9 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     const bool pair_ok = (dl_ok || i8_ok) && a->causal && pl.splits == 1 && 32 % G == 0;
     // (32 % G == 0 in pair_ok: G <= 32, so 32 / G >= 1)
     const long long pair_wgs = pair_ok ? pairs * (((a->max_query_len + 32 / G - 1) / (32 / G) + 1) / 2) : 0;
-    pl.r16 = pair_ok && (path == TI_PATH_PREFILL_PAIRED16 || (auto_path && R16_BY_DEFAULT && pair_wgs <= 512));
+    pl.r16 = pair_ok && (a->path == TI_PATH_PREFILL_PAIRED16 || (auto_path && R16_BY_DEFAULT && pair_wgs <= 512));
     pl.pair = pl.r16 || (pair_ok && dl_ok && pl.dl && pl.wpg == 2 && pl.ng == 4 &&
-                         (path == TI_PATH_PREFILL_PAIRED || (auto_path && PAIR_BY_DEFAULT)));
+                         (a->path == TI_PATH_PREFILL_PAIRED || (auto_path && PAIR_BY_DEFAULT)));
     if (pl.pair) {
         pl.TQ = 32 / G;
         pl.qtiles = (a->max_query_len + pl.TQ - 1) / pl.TQ;
