@@ -48,6 +48,16 @@ CASES = {
 def test_prefill_form(gpu, name):
     """Also with NaN in every pool row (INT8: scale) that no sequence holds, which tiles past a
     step's last key read: none may reach the output."""
+    run_case(name, ti.TI_PATH_AUTO)
+
+
+@pytest.mark.parametrize("name", ["ksplit_int8_ragged", "solo_int8", "solo_int8_d64"])
+def test_prefill_int8_stale_scales(gpu, name):
+    """The same through the four-wave kernel, which takes the INT8 steps that no form above does."""
+    run_case(name, ti.TI_PATH_PREFILL_STAGED)
+
+
+def run_case(name, path):
     kind, D, H, KVH, P, seqs, causal = CASES[name]
     g = rng(5200 + list(CASES).index(name))
     used = [-(-(s + n) // P) for s, n in seqs]
@@ -84,9 +94,10 @@ def test_prefill_form(gpu, name):
         v[stale] = float("nan")
     out = torch.full_like(qd, float("nan"))
     print(f"case {name}", flush=True)
-    ws = ti.attention_workspace(BE, qd, k, num_seqs=len(seqs), max_query_len=nmax)
+    ws = ti.attention_workspace(BE, qd, k, num_seqs=len(seqs), max_query_len=nmax, path=path)
     ti.paged_attention_(BE, out, ws, qd, k, v, torch.from_numpy(bts).cuda(), torch.from_numpy(positions).cuda(), scale,
-                        causal, query_start_loc=torch.from_numpy(qsl).cuda() if len(seqs) > 1 else None, max_query_len=nmax)
+                        causal, query_start_loc=torch.from_numpy(qsl).cuda() if len(seqs) > 1 else None, max_query_len=nmax,
+                        path=path)
     got = out.float().cpu().numpy()
     for b, (s, n) in enumerate(seqs):
         if n == 0:

@@ -264,8 +264,10 @@ __device__ __forceinline__ void store_tile(const Stage<D, INT8, GT> &st, Smem<D>
         }
     }
     if (INT8 && gtid < 2 * KT) {
-        if (gtid < KT) sm.sk[buf][gtid] = st.s;
-        else sm.sv[buf][gtid - KT] = st.s;
+        // scales of keys past the step's end may hold any bits too (a NaN one times p = 0 is NaN)
+        const float s = gtid % KT < valid_keys ? st.s : 0.0f;
+        if (gtid < KT) sm.sk[buf][gtid] = s;
+        else sm.sv[buf][gtid - KT] = s;
     }
 }
 
