@@ -173,6 +173,15 @@ def test_pinned_prefill_variants_keep_their_plan():
         assert ws(a, _cache()) == (_lib.TI_OK, want), path
 
 
+def test_block_steps_keep_their_key_splits():
+    """AUTO leaves launches of fewer than 256 64-row q-tiles to the four-wave plan, which splits
+    their keys in two (the query does not know the tables' width): blocks of up to 64 packed
+    rows for 17 to 23 sequences, and 6 sequences of three 128-row q-tiles."""
+    for n, seqs in ((16, 17), (9, 23), (66, 6)):
+        a = _args(num_seqs=seqs, max_query_len=n, total_tokens=seqs * n)
+        assert ws(a, _cache()) == (_lib.TI_OK, seqs * 8 * 2 * 4 * n * 130 * 4), (n, seqs)
+
+
 def test_store_rope_inputs_validation():
     L = ti.load_library()
     c = _cache()

@@ -105,3 +105,73 @@ def run_case(name, path):
         ref = orc.attention(q[qsl[b]:qsl[b + 1]], bts[b], s, scale, causal, **pools)
         excess = np.abs(ref - got[qsl[b]:qsl[b + 1]]) - (2e-2 + (np.abs(ref) * 2.0 ** -8 if kind == "int8" else 0))
         assert float(np.max(excess)) <= 0, f"sequence {b}: over the tolerance by {np.max(excess)}"
+
+
+# name: (cache, heads, sequences (start, n), block-table width in positions (0: just wide enough),
+#        the pinned path whose kernel AUTO takes, or None: a form of the ping-pong kernel)
+STAGED, PAIRED16 = ti.TI_PATH_PREFILL_STAGED, ti.TI_PATH_PREFILL_PAIRED16
+ragged5 = [(831 + 300 * b, 37 + 20 * b) for b in range(5)]
+PICKS = {
+    # blocks of one q-tile per sequence: key splits, or the 16-row kernel where keys do not split
+    "block_17_wide": ("bf16", 32, [(300, 16)] * 17, 2064, STAGED),
+    "block_17_narrow": ("bf16", 32, [(300, 16)] * 17, 0, PAIRED16),
+    "block_17_1040": ("bf16", 32, [(300, 16)] * 17, 1040, None),
+    "block_23_wide": ("bf16", 32, [(40 * b, 16 - b % 8) for b in range(23)], 4096, STAGED),
+    "block_24_wide": ("bf16", 32, [(40 * b, 16 - b % 8) for b in range(24)], 4096, None),
+    "block_32": ("bf16", 32, [(40 * (b % 9), 16) for b in range(32)], 2064, PAIRED16),
+    "block_63": ("bf16", 32, [(40 * (b % 9), 16) for b in range(63)], 0, PAIRED16),
+    "block_64": ("bf16", 32, [(40 * (b % 9), 16) for b in range(64)], 0, None),
+    "block_int8_32": ("int8", 32, [(40 * (b % 9), 16) for b in range(32)], 2064, PAIRED16),
+    "block_int8_64": ("int8", 32, [(40 * (b % 9), 16) for b in range(64)], 0, PAIRED16),
+    "block_int8_65": ("int8", 32, [(40 * (b % 9), 16) for b in range(65)], 0, None),
+    # few q-tiles per sequence
+    "three_tiles_narrow": ("bf16", 32, [(60, 66)] * 6, 0, PAIRED16),
+    "three_tiles_1040": ("bf16", 32, [(60, 66)] * 6, 1040, None),
+    "int8_20x40": ("int8", 32, [(70, 40)] * 20, 2064, PAIRED16),
+    "int8_ragged": ("int8", 32, ragged5, 4096, PAIRED16),
+    "int8_short_beyond_one_round": ("int8", 32, [(9, 180)] * 7, 0, None),
+    "short_beyond_one_round": ("bf16", 32, [(b, 123 + 10 * b) for b in range(6)], 0, None),
+    "g3_late_start": ("bf16", 24, [(0, 850)], 0, PAIRED16),
+    "g3_first": ("bf16", 24, [(0, 890)], 0, None),
+}
+
+
+@pytest.mark.parametrize("name", list(PICKS))
+def test_prefill_pick(gpu, name):
+    """The kernel AUTO takes on each side of the pick's lines, by bit-equality with the pinned one
+    (whose MFMA shape or order of key tiles no ping-pong form shares), and its result on the first
+    and the last sequence."""
+    kind, H, seqs, width, like = PICKS[name]
+    D, KVH, P, B = 128, 8, 16, len(seqs)
+    g = rng(5400 + list(PICKS).index(name))
+    used = [-(-(s + n) // P) for s, n in seqs]
+    pages, nmax = sum(used) + 1, max(n for _, n in seqs)
+    bts = np.zeros((B, max(width // P, max(used))), np.int32)
+    ids = iter(g.permutation(pages) + 1)
+    for b in range(B):
+        bts[b, :used[b]] = [next(ids) for _ in range(used[b])]
+    qsl = np.concatenate([[0], np.cumsum([n for _, n in seqs])]).astype(np.int32)
+    q = randn(g, qsl[-1], H, D, bf16=True)
+    kp, vp = randn(g, pages, KVH, P, D, bf16=True), randn(g, pages, KVH, P, D, bf16=True)
+    k, v = torch.from_numpy(kp).bfloat16().cuda(), torch.from_numpy(vp).bfloat16().cuda()
+    pools = dict(k_pages=kp, v_pages=vp)
+    if kind == "int8":
+        flat = [x.transpose(1, 2).reshape(-1, KVH, D).contiguous() for x in (k, v)]
+        k, v = ti.int8_kv_pools(D, P, KVH, pages)
+        ti.store_kv_(BE, k, v, *flat, torch.arange(1, P * pages + 1, dtype=torch.int32, device="cuda"))
+        pools = dict(layer_q=k.layer_q.cpu().numpy(), layer_scale=k.layer_scale.cpu().numpy(), smooth=np.ones(D, np.float32))
+    qd, scale = torch.from_numpy(q).bfloat16().cuda(), 1 / math.sqrt(D)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in seqs]).to(torch.int32).cuda()
+    outs = []
+    for path in (ti.TI_PATH_AUTO, like or (PAIRED16 if kind == "int8" else STAGED)):
+        print(f"pick {name} path {path}", flush=True)
+        ws = ti.attention_workspace(BE, qd, k, num_seqs=B, max_query_len=nmax, path=path)
+        outs.append(torch.full_like(qd, float("nan")))
+        ti.paged_attention_(BE, outs[-1], ws, qd, k, v, torch.from_numpy(bts).cuda(), pos, scale,
+                            query_start_loc=torch.from_numpy(qsl).cuda(), max_query_len=nmax, path=path)
+    assert torch.equal(*outs) == (like is not None)
+    got = outs[0].float().cpu().numpy()
+    for b in (0, B - 1):
+        ref = orc.attention(q[qsl[b]:qsl[b + 1]], bts[b], seqs[b][0], scale, True, **pools)
+        excess = np.abs(ref - got[qsl[b]:qsl[b + 1]]) - (2e-2 + (np.abs(ref) * 2.0 ** -8 if kind == "int8" else 0))
+        assert float(np.max(excess)) <= 0, f"sequence {b}: over the tolerance by {np.max(excess)}"

@@ -169,8 +169,9 @@ struct ti_prefill_plan {
 ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c, bool bound_keys);
 int ti_launch_prefill(const ti_attention_args *a, const ti_kv_cache *c, const ti_prefill_plan &p,
                       hipStream_t s);
-// The ping-pong form a prefill on `path` takes (AUTO, PREFILL: the library's pick).
-int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path);
+// The ping-pong form a prefill on `path` takes (AUTO, PREFILL: the library's pick; bound_keys as
+// in ti_plan_prefill).
+int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path, bool bound_keys);
 int ti_launch_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, const ti_prefill_plan &p,
                          hipStream_t s);
 // fp32 path: its key splits and workspace bytes (host shapes only).

@@ -1229,7 +1229,7 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     const long long pairs = (long long)c->kv_heads * a->num_seqs;
     const long long key_tiles = ((long long)a->block_table_stride * c->page_size + 31) / 32;
     const bool auto_path = a->path == TI_PATH_PREFILL || a->path == TI_PATH_AUTO;
-    pl.pp = ti_pick_prefill_pp(a, c, a->path);
+    pl.pp = ti_pick_prefill_pp(a, c, a->path, bound_keys);
     pl.dl = 0;
     pl.pair = 0;
     pl.r16 = 0;

@@ -608,43 +608,77 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 
 // The ping-pong kernel takes bf16 activations over dense or INT8 caches with head_dim 64 or
 // 128, power-of-two pages of at least 16 tokens (a page of all KV heads under 4 GiB: 32-bit
-// strides) and at most 128 heads per KV head.
+// strides) and at most 64 heads per KV head (as every prefill kernel).
 //
-// The library's pick counts the launch's 128-row work-groups, W (head counts 32 / 8 unless
-// stated; each figure: this form against the kernel that takes the step otherwise, the
-// four-wave or the 16-row paired one, same process, graph replays, inputs warm):
-//   W <= 128: none. A work-group's fixed cost (about 7 us: first loads, merge, stores) and
-//     idle CUs outweigh the faster steps (512 tokens, W = 128: the 16-row kernel's one round of
-//     256 work-groups takes 9.3 us).
+// The library's pick counts the launch's 128-row work-groups, W; its 64-row ones, q64, the
+// four-wave plan's on small launches; and the 32-key tiles that a block table has room for
+// (nothing else on the host bounds the contexts). Head counts 32 / 8 unless stated; each figure:
+// this form against the kernel that takes the step otherwise, the four-wave or the 16-row paired
+// one, same process, graph replays, keys from HBM. A KSPLIT work-group has a CU to itself and
+// costs about 7 us beside its steps (first loads, merge, stores), so it wins where those steps
+// are many and loses where half its rows are padding or a second round is short; SOLO, which
+// shares a CU, is the form for short steps of more than one round.
+//   W <= 128: none (512 tokens: the 16-row kernel's one round of 256 takes 9.3 us).
+//   q64 < 256: none. From 32 tiles the four-wave plan's key splits even out ragged contexts (17 x
+//     16 tokens on 500 to 4000: 46 us, KSPLIT 57); below, unsplit, it is the 16-row kernel (17 x
+//     16 on 200 9.9, KSPLIT 11.3; 6 x 66 from scratch 7.8, 9.8). But KSPLIT from 32 to 40 tiles
+//     (17 x 16 on 700 19.3 against 29.2), and from W = 192 (24 x 16 on 4096 75.7 against 97.4,
+//     ragged to 4000 61 against 67; to 8000 120 against 115).
+//   One q-tile of up to 64 rows per sequence: none for W < 512, the 16-row kernel's range (32 x
+//     16 on 4096 KSPLIT 98.9 against 91.8, on 200 12.6 against 11.2; INT8 107 against 72, at 64 x
+//     16 SOLO 196 against 150). From there SOLO (96 x 16 on 200 31.0 against 39.8).
+//   INT8 whose 64-row work-groups fit that range: none (20 x 40 on 1000 KSPLIT 64
+//     against 42). Nor for W <= 256, counted by the tokens the sequences hold (5 prompts of 37 to
+//     119 on 800 to 2800 68 against 50): converting tiles doubles the staging there. Beyond, with
+//     few idle rows, KSPLIT (1500 on 4096 206 against 232), but at head_dim 64 only alone (20
+//     x 95 on 3000 142 against 130).
 //   W <= 512: KSPLIT. At most two work-groups per CU, one resident at a time, each with half
-//     the steps of an unsplit q-tile: 520 tokens 14.4 against 15.8 us, 1024 22.5 against
-//     26.1, 2048 47.2 against 56.5; 576 on 2000 40.7 against 65.2; D = 64, 1024 15.1 against
-//     21.4. INT8 tiles cost twice the staging there, and single prompts start later: 1024
-//     tokens (W = 256) 31.1 against 29.8, 1280 37.0 against 40.3. So do q-tiles with rows to
-//     spare (G = 3: 768 tokens, W = 152, 18.1 against 17.7).
+//     the steps of an unsplit q-tile: 520 tokens 15.5 against 16.9 us, 1000 22.5 against 26.2,
+//     2000 46.6 against 55.4; 600 on 4096 65.9 against 114.8; D = 64, 1000 15.6 against 21.8.
+//     q-tiles with rows to spare start later (G = 3: 800 tokens, W = 160, 19.4 against 18.4),
+//     D = 64 by the tokens held (5 chunks of 37 to 119 on 800 to 2800 31.3 against 29.1).
+//     Below 32 tiles and past one round SOLO (12 x 90 tokens 12.6, KSPLIT 19.0, four-wave 18.0;
+//     eight of 256, D = 64, 11.8, 16.0, 14.9).
 //   more: SHARED for dense D = 128 (half the loads and LDS stores per row): 3072 tokens 85.0
 //     against 118.7 us, 8192 493 against 539; else SOLO, whose work-groups share a CU (two,
 //     D = 64 three) and hide each other's fixed cost: INT8 3072 tokens 110.8 against 145.8,
 //     D = 64 8192 309 against 394, eight D = 64 prompts of 100 to 2000 tokens 58.8 against
 //     78.3. SOLO also takes dense batches of short sequences, whose 256-row tiles are mostly
 //     padding: 16 prompts of 30 to 300 tokens 22.1 us, SHARED 25.3, 28.2 before.
-//   At most two q-tiles per sequence (T <= 2): SOLO from W = 512 (32 x 60 tokens from scratch
-//     / on 2000: 0.76 / 0.84 of the time), KSPLIT at D = 128 dense (9 x 60: 0.75), INT8 from 256.
-int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path) {
+// Of 3177 shapes on either side of these lines, of up to 128 sequences, uniform and ragged, seven
+// are more than 3 % slower than on the kernels that took them before this one had forms, by at
+// most 6 % (INT8 prompts whose tables have just 33 tiles).
+int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path, bool bound_keys) {
     const int G = a->q_heads / c->kv_heads, P = c->page_size, D = c->head_dim;
-    if (a->dtype != TI_BF16 || (D != 64 && D != 128) || P < 16 || (P & (P - 1)) || G > 128 ||
+    if (a->dtype != TI_BF16 || (D != 64 && D != 128) || P < 16 || (P & (P - 1)) || G > 64 ||
         2ull * c->kv_heads * P * D > 0xffffffffull)
         return TI_PP_NONE;
     const bool dense = c->kind == TI_KV_DENSE, dense128 = dense && D == 128;
     if (path == TI_PATH_PREFILL_PINGPONG && dense128 && 256 % G == 0) return TI_PP_SHARED;
     if (path != TI_PATH_AUTO && path != TI_PATH_PREFILL) return TI_PP_NONE;
-    const long long TQ = 128 / G, T = (a->max_query_len + TQ - 1) / TQ, W = T * c->kv_heads * a->num_seqs;
+    const long long pairs = (long long)c->kv_heads * a->num_seqs, n = a->max_query_len;
+    const long long TQ = 128 / G, T = (n + TQ - 1) / TQ, q64 = (n + 64 / G - 1) / (64 / G) * pairs;
     // grids hold 65535 q-tiles: 256-row ones where those have been taken, none where not
     if (T > 65535) return dense128 && 256 % G == 0 ? TI_PP_SHARED : TI_PP_NONE;
-    if (T <= 2) return W >= 512 ? TI_PP_SOLO : (D == 128 && W >= (dense ? 129 : 256) ? TI_PP_KSPLIT : TI_PP_NONE);
-    const int first = dense ? (128 % G == 0 ? 129 : 160) : (a->num_seqs > 1 ? 160 : D == 64 ? 256 : 257);
-    if (W < first) return TI_PP_NONE;
-    if (W <= 512) return TI_PP_KSPLIT;
+    long long W = T * pairs;
+    const long long tiles = bound_keys ? ((long long)a->block_table_stride * P + 31) / 32 : 1LL << 40;
+    // Only here does the four-wave plan split keys, and only from 32 tiles: a workspace query
+    // (unbounded tiles) that answers KSPLIT is right for narrower tables too.
+    if (q64 < 256)
+        return dense && (dense128 || T > 2) && tiles >= 32 && W >= (tiles <= 40 ? 129 : 192) ? TI_PP_KSPLIT : TI_PP_NONE;
+    if (T == 1 && q64 == W && W < (dense ? 512 : 513)) return TI_PP_NONE;
+    if (!dense && W > 256 && q64 <= 512) return TI_PP_NONE;
+    const int short_form = tiles < 32 && W > 256 ? TI_PP_SOLO : TI_PP_KSPLIT;
+    if (T <= 2) return W >= 512 ? TI_PP_SOLO : (D == 128 && W >= (dense ? 129 : 256) ? short_form : TI_PP_NONE);
+    const long long held = W * a->total_tokens / (n * a->num_seqs);
+    if (!dense) {
+        if (W <= 640) W = held;
+        if (W < (D == 64 && a->num_seqs == 1 ? 256 : 257)) return TI_PP_NONE;
+        if (W > 512 || tiles < 32) return TI_PP_SOLO;
+        return D == 128 || a->num_seqs == 1 ? TI_PP_KSPLIT : TI_PP_NONE;
+    }
+    if ((D == 64 && W <= 512 ? held : W) < (128 % G == 0 ? 129 : tiles <= 40 ? 176 : 160)) return TI_PP_NONE;
+    if (W <= 512) return short_form;
     return dense128 && T > 6 && !(a->num_seqs >= 8 && W > 1024) ? TI_PP_SHARED : TI_PP_SOLO;
 }
 
