@@ -643,8 +643,11 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     against 118.7 us, 8192 493 against 539; else SOLO, whose work-groups share a CU (two,
 //     D = 64 three) and hide each other's fixed cost: INT8 3072 tokens 110.8 against 145.8,
 //     D = 64 8192 309 against 394, eight D = 64 prompts of 100 to 2000 tokens 58.8 against
-//     78.3. SOLO also takes dense batches of short sequences, whose 256-row tiles are mostly
-//     padding: 16 prompts of 30 to 300 tokens 22.1 us, SHARED 25.3, 28.2 before.
+//     78.3. SOLO also takes dense D = 128 batches whose sequences are short in queries and keys (16
+//     x 300 tokens 39.8 against 42.1 on SHARED, 16 x 512 71.9, 74.9) or mostly absent (a prompt of
+//     2000 beside 16 tokens 56.5, 65.4): 256-row tiles there are padding or have few steps. Not
+//     longer ones (SOLO, SHARED: 8 x 1024 102, 100; 8 x 2048 331, 306; 8 x 4096 1163, 1041; 16 x
+//     512 on 4096 609, 534).
 // Of 3177 shapes on either side of these lines, of up to 128 sequences, uniform and ragged, seven
 // are more than 3 % slower than on the kernels that took them before this one had forms, by at
 // most 6 % (INT8 prompts whose tables have just 33 tiles).
@@ -679,7 +682,8 @@ int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int pat
     }
     if ((D == 64 && W <= 512 ? held : W) < (128 % G == 0 ? 129 : tiles <= 40 ? 176 : 160)) return TI_PP_NONE;
     if (W <= 512) return short_form;
-    return dense128 && T > 6 && !(a->num_seqs >= 8 && W > 1024) ? TI_PP_SHARED : TI_PP_SOLO;
+    const bool padded = a->num_seqs >= 8 && W > 1024 && ((T <= 24 && tiles <= 40) || 4 * held < W);
+    return dense128 && T > 6 && !padded ? TI_PP_SHARED : TI_PP_SOLO;
 }
 
 int ti_launch_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, const ti_prefill_plan &pl,
