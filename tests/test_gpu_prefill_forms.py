@@ -13,24 +13,26 @@ import torch
 import tileinfer_hip as ti
 from helpers import randn, rng, smoothing
 from oracle import oracle as orc
+from test_prefill_pick import KSPLIT, NONE, SHARED, SOLO, pick
 
 pytestmark = pytest.mark.gpu
 BE = ti.HipBackend()
 
-# name: (cache, D, heads, kv_heads, page_size, sequences (start, n), causal)
+# name (its first word is the form, others take the kernels outside this one): (cache, D, heads,
+# kv_heads, page_size, sequences (start, n), causal[, block-table width in positions])
 CASES = {
     "paired16_ragged": ("bf16", 128, 32, 8, 16, [(700, 40), (0, 130), (0, 0)], True),   # W = 120: none
     "ksplit_dense_first": ("bf16", 128, 32, 8, 16, [(0, 520)], True),            # W = 136
     "ksplit_dense_odd_tiles": ("bf16", 128, 32, 8, 64, [(33, 700)], True),
     "ksplit_dense_non_causal": ("bf16", 128, 32, 8, 16, [(77, 641)], False),
-    "ksplit_dense_g3": ("bf16", 128, 24, 8, 32, [(10, 850)], True),              # 42 positions a q-tile
-    "ksplit_dense_ragged": ("bf16", 128, 32, 8, 16, [(700, 40), (0, 130), (0, 0), (900, 1), (5, 300)], True),
+    "ksplit_dense_g3": ("bf16", 128, 24, 8, 32, [(10, 850)], True, 2048),        # 42 positions a q-tile
+    "ksplit_dense_ragged": ("bf16", 128, 32, 8, 16, [(700, 40), (0, 130), (0, 0), (900, 1), (5, 300)], True, 2048),
     "ksplit_dense_two_tiles": ("bf16", 128, 32, 8, 16, [(60 * (b % 4), 33 + b) for b in range(16)], True),
     "ksplit_dense_d64": ("bf16", 64, 32, 8, 32, [(5, 700)], True),
     "ksplit_dense_d64_non_causal": ("bf16", 64, 16, 8, 16, [(100, 650), (0, 650)], False),
-    "ksplit_int8_first": ("int8", 128, 32, 8, 16, [(0, 1030)], True),            # W = 264
-    "ksplit_int8_ragged": ("int8", 128, 32, 8, 64, [(300, 299), (0, 31), (0, 0), (65, 300), (1, 1)], True),
-    "ksplit_int8_d64": ("int8", 64, 16, 8, 16, [(33, 640), (0, 600)], True),
+    "ksplit_int8_first": ("int8", 128, 32, 8, 16, [(0, 1030)], True, 2048),      # W = 264
+    "int8_ragged": ("int8", 128, 32, 8, 64, [(300, 299), (0, 31), (0, 0), (65, 300), (1, 1)], True),
+    "int8_d64": ("int8", 64, 16, 8, 16, [(33, 640), (0, 600)], True),
     "solo_dense_short": ("bf16", 128, 32, 8, 16, [(17 * b, 129 + b) for b in range(16)], True),
     "solo_dense_two_tiles": ("bf16", 128, 32, 8, 16, [(3 * b, 33 + b % 8) for b in range(32)], True),
     "solo_dense_d64": ("bf16", 64, 32, 8, 64, [(0, 700), (100, 300), (0, 0), (900, 650)], True),
@@ -41,6 +43,9 @@ CASES = {
     # an empty sequence in a step whose first position is 0: no key tile, no page to look up
     "paired16_empty_first": ("bf16", 128, 32, 8, 16, [(0, 0), (0, 130), (700, 40)], True),
     "paired16_int8_empty_first": ("int8", 128, 32, 8, 16, [(0, 0), (0, 130), (100, 40)], True),
+    "ksplit_int8_ragged": ("int8", 128, 32, 8, 64, [(300, 299), (0, 231), (0, 0), (65, 300), (1, 290)], True, 2048),
+    "ksplit_int8_d64": ("int8", 64, 32, 8, 16, [(33, 1040)], True, 2048),
+    "shared_dense_g3": ("bf16", 128, 24, 8, 32, [(5, 700), (0, 333), (930, 85), (0, 0)], True),   # 85 positions a q-tile
 }
 
 
@@ -48,22 +53,27 @@ CASES = {
 def test_prefill_form(gpu, name):
     """Also with NaN in every pool row (INT8: scale) that no sequence holds, which tiles past a
     step's last key read: none may reach the output."""
+    kind, D, H, KVH, P, seqs, _, width = (*CASES[name], 0)[:8]
+    forms = {"shared": SHARED, "ksplit": KSPLIT, "solo": SOLO}
+    assert forms.get(name.split("_")[0], NONE) == pick(
+        max(n for _, n in seqs), len(seqs), max(width, P * (max(-(-(s + n) // P) for s, n in seqs) + 2)),
+        sum(n for _, n in seqs), int(kind == "int8"), H, KVH, D, P)
     run_case(name, ti.TI_PATH_AUTO)
 
 
-@pytest.mark.parametrize("name", ["ksplit_int8_ragged", "solo_int8", "solo_int8_d64"])
+@pytest.mark.parametrize("name", ["int8_ragged", "solo_int8", "solo_int8_d64"])
 def test_prefill_int8_stale_scales(gpu, name):
     """The same through the four-wave kernel, which takes the INT8 steps that no form above does."""
     run_case(name, ti.TI_PATH_PREFILL_STAGED)
 
 
 def run_case(name, path):
-    kind, D, H, KVH, P, seqs, causal = CASES[name]
+    kind, D, H, KVH, P, seqs, causal, width = (*CASES[name], 0)[:8]
     g = rng(5200 + list(CASES).index(name))
     used = [-(-(s + n) // P) for s, n in seqs]
     pages, nmax = sum(used) + 3, max(n for _, n in seqs)
     perm = (g.permutation(pages) + 1).astype(np.int32)
-    bts = np.zeros((len(seqs), max(used) + 2), np.int32)
+    bts = np.zeros((len(seqs), max(max(used) + 2, width // P)), np.int32)
     rows = np.zeros((pages, P), bool)               # rows that hold a key
     at = 0
     for b, (s, n) in enumerate(seqs):

@@ -10,14 +10,14 @@ from tileinfer_hip import _lib
 NONE, SHARED, KSPLIT, SOLO = range(4)
 
 
-def pick(n, seqs, keys, total=None, kind=0, heads=32, kv_heads=8, D=128):
+def pick(n, seqs, keys, total=None, kind=0, heads=32, kv_heads=8, D=128, page=16):
     f = getattr(ti.load_library(), "_Z18ti_pick_prefill_ppPK17ti_attention_argsPK11ti_kv_cacheib")
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_bool]
     c = _lib.KVCache()
-    c.kind, c.head_dim, c.page_size, c.kv_heads, c.num_pages = kind, D, 16, kv_heads, 100
+    c.kind, c.head_dim, c.page_size, c.kv_heads, c.num_pages = kind, D, page, kv_heads, 100
     a = _lib.AttentionArgs()
     a.dtype, a.q_heads, a.num_seqs, a.max_query_len = _lib.TI_BF16, heads, seqs, n
-    a.total_tokens, a.block_table_stride = seqs * n if total is None else total, keys // 16
+    a.total_tokens, a.block_table_stride = seqs * n if total is None else total, keys // page
     a.scale, a.causal = 1.0, 1
     return f(ctypes.byref(a), ctypes.byref(c), _lib.TI_PATH_AUTO, True)
 
@@ -70,6 +70,9 @@ def test_pick_of_large_launches(want, kw):
     (KSPLIT, dict(n=1184, seqs=2, keys=4112, kind=1, total=1723)),
     (NONE, dict(n=1184, seqs=2, keys=4112, kind=1, total=1723, D=64)),
     (SOLO, dict(n=1184, seqs=2, keys=4112, kind=1)),
+    (NONE, dict(n=534, seqs=2, keys=1040, kind=1)),
+    (NONE, dict(n=534, seqs=2, keys=1280, kind=1)),
+    (KSPLIT, dict(n=534, seqs=2, keys=1296, kind=1)),
     # one round and more, with few key tiles and many
     (NONE, dict(n=512, seqs=1, keys=1040)),
     (KSPLIT, dict(n=520, seqs=1, keys=1040)),

@@ -201,7 +201,9 @@ __device__ __forceinline__ void load_tile(Stage<D, INT8, GT> &st, const PrefillP
             }
         }
         if (INT8 && gtid < 2 * KT) {
-            const int key = gtid % KT;
+            // keys past kend take the last key's scale: a stale one may be NaN, and p = 0 times NaN
+            // is NaN
+            const int key = min(gtid % KT, kend - 1 - kt * KT);
             const long long row = base[key >> 4] / D + (key & 15);
             st.s = gtid < KT ? p.ls[row] : p.ls[half_s + row];
         }
@@ -264,10 +266,8 @@ __device__ __forceinline__ void store_tile(const Stage<D, INT8, GT> &st, Smem<D>
         }
     }
     if (INT8 && gtid < 2 * KT) {
-        // scales of keys past the step's end may hold any bits too (a NaN one times p = 0 is NaN)
-        const float s = gtid % KT < valid_keys ? st.s : 0.0f;
-        if (gtid < KT) sm.sk[buf][gtid] = s;
-        else sm.sv[buf][gtid - KT] = s;
+        if (gtid < KT) sm.sk[buf][gtid] = st.s;
+        else sm.sv[buf][gtid - KT] = st.s;
     }
 }
 

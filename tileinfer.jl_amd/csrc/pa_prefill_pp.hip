@@ -630,8 +630,8 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //   INT8 whose 64-row work-groups fit that range: none (20 x 40 on 1000 KSPLIT 64
 //     against 42). Nor for W <= 256, counted by the tokens the sequences hold (5 prompts of 37 to
 //     119 on 800 to 2800 68 against 50): converting tiles doubles the staging there. Beyond, with
-//     few idle rows, KSPLIT (1500 on 4096 206 against 232), but at head_dim 64 only alone (20
-//     x 95 on 3000 142 against 130).
+//     few idle rows and more than 40 tiles, KSPLIT (1500 on 4096 206 against 232; two prompts of
+//     520 23.9 against 22.6), but at head_dim 64 only alone (20 x 95 on 3000 142 against 130).
 //   W <= 512: KSPLIT. At most two work-groups per CU, one resident at a time, each with half
 //     the steps of an unsplit q-tile: 520 tokens 15.5 against 16.9 us, 1000 22.5 against 26.2,
 //     2000 46.6 against 55.4; 600 on 4096 65.9 against 114.8; D = 64, 1000 15.6 against 21.8.
@@ -648,9 +648,10 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     2000 beside 16 tokens 56.5, 65.4): 256-row tiles there are padding or have few steps. Not
 //     longer ones (SOLO, SHARED: 8 x 1024 102, 100; 8 x 2048 331, 306; 8 x 4096 1163, 1041; 16 x
 //     512 on 4096 609, 534).
-// Of 3177 shapes on either side of these lines, of up to 128 sequences, uniform and ragged, seven
-// are more than 3 % slower than on the kernels that took them before this one had forms, by at
-// most 6 % (INT8 prompts whose tables have just 33 tiles).
+// Over 3757 shapes on either side of these lines, of up to 128 sequences, uniform and ragged, steps
+// take 0.84 times as long in the mean as on the kernels that took them before this one had forms.
+// Slower by more than 3 %: 17, batches of W < 200 whose contexts are ragged, which the host
+// cannot see (7 x 66 on 200 to 930 21.8 against 18.5; 5 x 110 on 1000 each 23.6 against 36.0).
 int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path, bool bound_keys) {
     const int G = a->q_heads / c->kv_heads, P = c->page_size, D = c->head_dim;
     if (a->dtype != TI_BF16 || (D != 64 && D != 128) || P < 16 || (P & (P - 1)) || G > 64 ||
@@ -678,7 +679,7 @@ int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int pat
         if (W <= 640) W = held;
         if (W < (D == 64 && a->num_seqs == 1 ? 256 : 257)) return TI_PP_NONE;
         if (W > 512 || tiles < 32) return TI_PP_SOLO;
-        return D == 128 || a->num_seqs == 1 ? TI_PP_KSPLIT : TI_PP_NONE;
+        return tiles > 40 && (D == 128 || a->num_seqs == 1) ? TI_PP_KSPLIT : TI_PP_NONE;
     }
     if ((D == 64 && W <= 512 ? held : W) < (128 % G == 0 ? 129 : tiles <= 40 ? 176 : 160)) return TI_PP_NONE;
     if (W <= 512) return short_form;
