@@ -254,5 +254,11 @@ PyMODINIT_FUNC PyInit__calls() {
     n_smooth = PyUnicode_InternFromString("smooth");
     n_half = PyUnicode_InternFromString("half");
     n_cos_sin = PyUnicode_InternFromString("cos_sin");
-    return PyModule_Create(&module);
+    PyObject *m = PyModule_Create(&module);
+    // the torch and Python whose layouts this was compiled for; _lib.py compares
+    if (m && PyModule_AddStringConstant(m, "built_for", BUILT_FOR) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }

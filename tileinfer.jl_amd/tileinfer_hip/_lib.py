@@ -8,6 +8,8 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libtileinfer_hip.so")
@@ -84,15 +86,30 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
 calls = None
 
 
+class _NoCalls:
+    """Stands in for _calls.so: leaves every call to backend.py's ctypes path."""
+
+    def __getattr__(self, name):
+        return lambda *args: -1
+
+
 def _bind_calls(L: ctypes.CDLL) -> None:
-    """Point the native call path (_calls.so) at the loaded library's entry points."""
+    """Point the native call path (_calls.so) at the loaded library's entry points. It only saves
+    host time: without it (not built, or for another torch or Python) every op goes through
+    ctypes, with a warning."""
     global calls
+    import torch
     from .kv import Int8Pages
+    here = f"torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]}"
     try:
         from . import _calls
+        if _calls.built_for != here:
+            raise ImportError(f"built for {_calls.built_for}, not for {here}")
     except ImportError as e:
-        raise RuntimeError("tileinfer_hip/_calls.so is missing or does not fit this torch: "
-                           "build it with `python tileinfer.jl_amd/build.py`") from e
+        warnings.warn(f"tileinfer_hip/_calls.so is not used ({e}): calls go through ctypes, about 6 us slower each; "
+                      "build it with `python tileinfer.jl_amd/build.py`", RuntimeWarning, stacklevel=2)
+        calls = _NoCalls()
+        return
     _calls.bind(Int8Pages, *(ctypes.cast(f, ctypes.c_void_p).value for f in
                              (L.ti_attention, L.ti_attention_inputs, L.ti_store_kv, L.ti_rope, L.ti_rmsnorm)))
     calls = _calls

@@ -2,8 +2,9 @@
 
 Each function mirrors one method of the reference for its TileBackend (same name with `!`
 spelled as a trailing `_`, same argument order and meaning) and calls one entry point of
-libtileinfer_hip.so through ctypes. torch tensors only carry device memory and the
-current stream; all compute is in the HIP library, and there is no fallback: if the
+libtileinfer_hip.so, from the native call path (_calls.so) where the arguments are plain
+ones, else through ctypes after the checks below. torch tensors only carry device memory and
+the current stream; all compute is in the HIP library, and there is no fallback: if the
 library is missing, the first call raises.
 
 Shapes are C order (the reference's column-major shapes reversed):
