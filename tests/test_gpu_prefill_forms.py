@@ -139,8 +139,9 @@ PICKS = {
     "three_tiles_1040": ("bf16", 32, [(60, 66)] * 6, 1040, None),
     "int8_20x40": ("int8", 32, [(70, 40)] * 20, 2064, PAIRED16),
     "int8_ragged": ("int8", 32, ragged5, 4096, PAIRED16),
-    "int8_short_beyond_one_round": ("int8", 32, [(9, 180)] * 7, 0, None),
-    "short_beyond_one_round": ("bf16", 32, [(b, 123 + 10 * b) for b in range(6)], 0, None),
+    "int8_short_beyond_one_round": ("int8", 32, [(9, 180)] * 7, 0, STAGED),
+    "short_beyond_one_round": ("bf16", 32, [(b, 123 + 10 * b) for b in range(6)], 0, STAGED),
+    "short_of_nine_tiles": ("bf16", 32, [(b, 257 + 10 * b) for b in range(4)], 0, None),
     "g3_late_start": ("bf16", 24, [(0, 850)], 0, PAIRED16),
     "g3_first": ("bf16", 24, [(0, 890)], 0, None),
 }

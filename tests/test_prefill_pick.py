@@ -60,6 +60,9 @@ def test_pick_of_large_launches(want, kw):
     (NONE, dict(n=16, seqs=63, keys=4112)),
     (SOLO, dict(n=16, seqs=64, keys=4112)),
     (KSPLIT, dict(n=17, seqs=32, keys=4112)),
+    (KSPLIT, dict(n=32, seqs=48, keys=48)),
+    (NONE, dict(n=32, seqs=48, keys=48, kind=1)),
+    (KSPLIT, dict(n=32, seqs=48, keys=4112, kind=1)),
     (NONE, dict(n=16, seqs=64, keys=4112, kind=1)),
     (SOLO, dict(n=16, seqs=65, keys=4112, kind=1)),
     # INT8: the 16-row kernel's range, tokens held
@@ -77,9 +80,10 @@ def test_pick_of_large_launches(want, kw):
     (NONE, dict(n=512, seqs=1, keys=1040)),
     (KSPLIT, dict(n=520, seqs=1, keys=1040)),
     (KSPLIT, dict(n=128, seqs=8, keys=144)),
-    (SOLO, dict(n=90, seqs=12, keys=144)),
+    (NONE, dict(n=90, seqs=12, keys=144)),
     (KSPLIT, dict(n=90, seqs=12, keys=4112)),
-    (SOLO, dict(n=256, seqs=8, keys=272, D=64)),
+    (NONE, dict(n=256, seqs=8, keys=272, D=64)),
+    (KSPLIT, dict(n=257, seqs=7, keys=272, D=64)),
     (KSPLIT, dict(n=256, seqs=8, keys=4112, D=64)),
     (NONE, dict(n=119, seqs=5, keys=4112, total=357, D=64)),
     (KSPLIT, dict(n=119, seqs=5, keys=4112, D=64)),

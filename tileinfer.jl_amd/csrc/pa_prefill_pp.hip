@@ -616,8 +616,7 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 // this form against the kernel that takes the step otherwise, the four-wave or the 16-row paired
 // one, same process, graph replays, keys from HBM. A KSPLIT work-group has a CU to itself and
 // costs about 7 us beside its steps (first loads, merge, stores), so it wins where those steps
-// are many and loses where half its rows are padding or a second round is short; SOLO, which
-// shares a CU, is the form for short steps of more than one round.
+// are many and loses where half its rows are padding or a second round is short.
 //   W <= 128: none (512 tokens: the 16-row kernel's one round of 256 takes 9.3 us).
 //   q64 < 256: none. From 32 tiles the four-wave plan's key splits even out ragged contexts (17 x
 //     16 tokens on 500 to 4000: 46 us, KSPLIT 57); below, unsplit, it is the 16-row kernel (17 x
@@ -637,8 +636,8 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     2000 46.6 against 55.4; 600 on 4096 65.9 against 114.8; D = 64, 1000 15.6 against 21.8.
 //     q-tiles with rows to spare start later (G = 3: 800 tokens, W = 160, 19.4 against 18.4),
 //     D = 64 by the tokens held (5 chunks of 37 to 119 on 800 to 2800 31.3 against 29.1).
-//     Below 32 tiles and past one round SOLO (12 x 90 tokens 12.6, KSPLIT 19.0, four-wave 18.0;
-//     eight of 256, D = 64, 11.8, 16.0, 14.9).
+//     Below 32 tiles and past one round only sequences of more than 8 q-tiles have the steps
+//     (four of 138 to 403 14.5 against 16.3; 12 x 90 19.0, 18.0; D = 64 8 x 256 16.0, 14.9).
 //   more: SHARED for dense D = 128 (half the loads and LDS stores per row): 3072 tokens 85.0
 //     against 118.7 us, 8192 493 against 539; else SOLO, whose work-groups share a CU (two,
 //     D = 64 three) and hide each other's fixed cost: INT8 3072 tokens 110.8 against 145.8,
@@ -649,9 +648,9 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     longer ones (SOLO, SHARED: 8 x 1024 102, 100; 8 x 2048 331, 306; 8 x 4096 1163, 1041; 16 x
 //     512 on 4096 609, 534).
 // Over 3757 shapes on either side of these lines, of up to 128 sequences, uniform and ragged, steps
-// take 0.84 times as long in the mean as on the kernels that took them before this one had forms.
-// Slower by more than 3 %: 17, batches of W < 200 whose contexts are ragged, which the host
-// cannot see (7 x 66 on 200 to 930 21.8 against 18.5; 5 x 110 on 1000 each 23.6 against 36.0).
+// take 0.87 times as long in the mean as on the kernels that took them before this one had forms.
+// Slower by more than 3 %: 15, nearly all batches of W < 200 whose contexts are ragged, which the
+// host cannot see (7 x 66 on 200 to 930 21.8 against 18.4; 5 x 110 on 1000 each 23.6 against 36.0).
 int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path, bool bound_keys) {
     const int G = a->q_heads / c->kv_heads, P = c->page_size, D = c->head_dim;
     if (a->dtype != TI_BF16 || (D != 64 && D != 128) || P < 16 || (P & (P - 1)) || G > 64 ||
@@ -672,17 +671,18 @@ int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int pat
         return dense && (dense128 || T > 2) && tiles >= 32 && W >= (tiles <= 40 ? 129 : 192) ? TI_PP_KSPLIT : TI_PP_NONE;
     if (T == 1 && q64 == W && W < (dense ? 512 : 513)) return TI_PP_NONE;
     if (!dense && W > 256 && q64 <= 512) return TI_PP_NONE;
-    const int short_form = tiles < 32 && W > 256 ? TI_PP_SOLO : TI_PP_KSPLIT;
-    if (T <= 2) return W >= 512 ? TI_PP_SOLO : (D == 128 && W >= (dense ? 129 : 256) ? short_form : TI_PP_NONE);
+    if (T <= 2 && W >= 512) return TI_PP_SOLO;
+    if (tiles < 32 && W > 256 && W <= 512 && (T > 1 || !dense) && T <= 8) return TI_PP_NONE;
+    if (T <= 2) return D == 128 && W >= (dense ? 129 : 256) ? TI_PP_KSPLIT : TI_PP_NONE;
     const long long held = W * a->total_tokens / (n * a->num_seqs);
     if (!dense) {
         if (W <= 640) W = held;
         if (W < (D == 64 && a->num_seqs == 1 ? 256 : 257)) return TI_PP_NONE;
-        if (W > 512 || tiles < 32) return TI_PP_SOLO;
+        if (W > 512) return TI_PP_SOLO;
         return tiles > 40 && (D == 128 || a->num_seqs == 1) ? TI_PP_KSPLIT : TI_PP_NONE;
     }
     if ((D == 64 && W <= 512 ? held : W) < (128 % G == 0 ? 129 : tiles <= 40 ? 176 : 160)) return TI_PP_NONE;
-    if (W <= 512) return short_form;
+    if (W <= 512) return TI_PP_KSPLIT;
     const bool padded = a->num_seqs >= 8 && W > 1024 && ((T <= 24 && tiles <= 40) || 4 * held < W);
     return dense128 && T > 6 && !padded ? TI_PP_SHARED : TI_PP_SOLO;
 }
