@@ -258,14 +258,16 @@ def test_attention_inputs_out_of_range(gpu, D, int8):
 
 
 # (dtype, INT8 cache, D, heads, kv_heads, tokens): both sides of the rules of the fused kernel's
-# layout (lanes of 16 elements from 5 * 256 * 1024 of them, 256 tokens, 8192 waves), head counts
+# layout (lanes of 16 elements from 5 * 256 * 1024 of them, at D = 64 2^24; 256 tokens; 8192 waves), head counts
 # that fill its waves or not, tokens that take several work-groups.
 LAYOUT_CASES = [(True, False, 128, 32, 8, 255), (True, False, 128, 32, 8, 256), (True, False, 128, 32, 4, 300),
                 (True, False, 128, 64, 8, 257), (True, False, 128, 3, 1, 256), (True, False, 64, 24, 8, 256),
                 (True, False, 64, 32, 8, 511), (True, False, 64, 32, 8, 512), (True, False, 128, 32, 8, 1638),
                 (True, False, 128, 32, 8, 1639), (True, True, 128, 32, 8, 820), (False, False, 128, 16, 8, 1366),
                 (True, False, 64, 5, 5, 301), (True, False, 64, 96, 8, 255), (True, True, 128, 32, 8, 256),
-                (True, True, 64, 32, 4, 270), (False, False, 128, 16, 8, 256), (False, True, 64, 12, 4, 3)]
+                (True, True, 64, 32, 4, 270), (False, False, 128, 16, 8, 256), (False, True, 64, 12, 4, 3),
+                (True, False, 64, 96, 8, 2520), (True, False, 64, 96, 8, 2521), (True, False, 64, 24, 8, 2048),
+                (True, True, 128, 12, 4, 2048), (True, True, 128, 32, 8, 819)]
 
 
 @pytest.mark.parametrize("norm", [False, True])

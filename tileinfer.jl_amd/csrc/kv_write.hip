@@ -665,19 +665,24 @@ static void launch_inputs(void *q_out, const ti_kv_cache *c, const void *qkv, co
         // fewer a lane's chain of shuffles and roundings shows (64 tokens 3.1 against 3.7 us, 300
         // of 16 / 8 heads 4.0 against 4.2). INT8 takes four, since its quantization divides element
         // by element (1500 tokens 12.3 against 13.4), and so do D = 128 tokens that would leave
-        // half a wave idle (36 heads, 2048 tokens: 11.5 against 11.9).
+        // half a wave idle (36 heads, 2048 tokens: 11.5 against 11.9). At D = 64 a token's lanes fill
+        // its waves worse and 2^24 elements are the line (32 / 8 heads with the norm: 8192 tokens 25.4
+        // -> 23.9, but 1400 7.0 -> 7.6; 16 / 8, 3000 tokens 8.4 -> 9.2).
         const int heads = nq + c->kv_heads;
-        const bool wide = sizeof(T) == 2 && !INT8 && (long long)n * heads * c->head_dim >= 5ll * 256 * 1024 &&
+        const bool wide = sizeof(T) == 2 && !INT8 &&
+                          (long long)n * heads * c->head_dim >= (c->head_dim == 64 ? 1ll << 24 : 5ll * 256 * 1024) &&
                           (c->head_dim == 64 || heads % 8 == 0);
-        // Work-groups of one wave as long as all waves fit the chip at once (32 per CU), so that no
-        // CU gets a whole token more than another (300 tokens 5.2 -> 4.7 us, 1500 13.1 -> 11.8,
-        // INT8 700 8.5 -> 7.7, of 16 / 8 Float32 heads 300 4.6 -> 4.2); beyond, whole tokens in up
-        // to 512 threads (4000 tokens of 16 / 8 heads 17.0 against 17.7, Float32 27.2 against
-        // 30.4). Up to 255 tokens 128 threads (one token 2.75 against 2.85, 130 tokens 3.4
-        // against 3.5).
+        // Work-groups of one wave for fewer than 8192 waves, so that no CU gets a whole token more
+        // than another (300 tokens 5.2 -> 4.7 us, 1500 13.1 -> 11.8, INT8 700 8.5 -> 7.7, of 16 / 8
+        // Float32 heads 300 4.6 -> 4.2; a measured line: the kernels hold 20 to 32 waves per CU). Beyond,
+        // whole tokens in up to 512 threads for wide lanes and Float32 (4000 tokens of 16 / 8 heads 17.0
+        // against 17.7, Float32 27.2 against 30.4), else 256 (INT8 8192 tokens 48.5, with 320 threads
+        // 52.7; 24 / 8 heads 39.8, 512 threads 44.1). Up to 255 tokens or 1700 waves 128 threads (one
+        // token 2.75 against 2.85, 130 tokens 3.4 against 3.5; 256 of 16 / 8 heads 3.72, 64 threads 3.92).
         const int lanes = heads * c->head_dim / (wide ? 16 : 8);
-        const int most = n < 256 ? 128 : (long long)n * lanes < 64ll * 32 * 256 ? 64 : 512;
-        const int parts = (lanes + most - 1) / most, threads = ((lanes + parts - 1) / parts + 63) / 64 * 64;
+        const int most = n < 256 || (long long)n * lanes < 64ll * 1700 ? 128 : (long long)n * lanes < 64ll * 8192 ? 64 : 512;
+        const int parts = (lanes + most - 1) / most;
+        const int threads = most == 512 && sizeof(T) == 2 && !wide ? 256 : ((lanes + parts - 1) / parts + 63) / 64 * 64;
         const dim3 grid(n, (lanes + threads - 1) / threads);
 #define TI_INPUTS_V(DD, NE)                                                                        \
     attention_inputs_v_kernel<T, NORM, INT8, DD, NE><<<grid, threads, 0, s>>>(                     \
