@@ -1,6 +1,6 @@
-"""The forms of the ping-pong prefill kernel (pa_prefill_pp.hip) that the library picks from the
-launch's 128-row work-groups, W = q-tiles x KV heads x sequences: KSPLIT (two teams of waves
-on every other key tile), SOLO (one team) and SHARED, at the edges of their ranges, dense and
+"""The forms of the ping-pong prefill kernel (pa_prefill_pp.hip) that the library picks from a
+launch's work-groups (W of 128 rows: q-tiles x KV heads x sequences) and its tables' width:
+KSPLIT (two teams of waves on every other key tile), SOLO (one team) and SHARED, at the edges of their ranges, dense and
 INT8, head_dim 64 and 128, ragged batches with an empty sequence, heads per KV head that do not
 divide a q-tile. Tolerances against the double-accumulated oracle as everywhere: max abs
 <= 2e-2, for INT8 plus one bf16 unit of the reference value."""

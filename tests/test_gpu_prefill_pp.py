@@ -1,9 +1,9 @@
 """The 8-wave ping-pong prefill kernel (pa_prefill_pp.hip) against the oracle.
 
-AUTO takes it only for large grids (a 4096-token prefill); TI_PATH_PREFILL_PINGPONG pins it for
-every shape it accepts (bf16 dense cache, head_dim 128, power-of-two pages of >= 16
-tokens, heads per KV head dividing 256), so these cases cover its masks, ragged last
-tiles, key splits, the prologue with one or two key tiles and batched calls. Tolerance:
+TI_PATH_PREFILL_PINGPONG pins its 256-row form, which AUTO takes for large grids only (a
+4096-token prefill; test_gpu_prefill_forms.py has the other forms), for every shape it accepts
+(bf16 dense cache, head_dim 128, power-of-two pages of >= 16 tokens, heads per KV head
+dividing 256), so these cases cover its masks, ragged last tiles, key splits, the prologue with one or two key tiles and batched calls. Tolerance:
 max abs <= 2e-2 against the double-accumulated oracle, and <= 5 bf16 ulps (the
 reference's bound, test/ops/tile.jl:237-259) up to 512 query tokens, the longest step its
 cases hold: longer causal prefills round more probabilities to bf16 and both prefill

@@ -29,15 +29,17 @@
 //   SOLO    one team on 128 rows, one barrier a step; two work-groups (head_dim 64: three)
 //           share a CU and overlap each other's phases, first loads and stores.
 //
-// What bounds it. On a full chip, power: a loop of these MFMAs alone runs at 1.5-1.7 GHz (0.70
-// us a SHARED step, 8 waves x 16 MFMAs of 32 cycles, against 0.45 us on 8 CUs at 2.4 GHz), and
-// every instruction saved shows. A SHARED step takes 0.95 us at 8192 tokens (LDS reads of all
-// operands 128 KB a step at 256 B per cycle and CU: not the limit). The MFMA phase used to wait
-// for its operands: keys read in pairs just before their MFMAs, softmax phases carrying the
-// staging. With the keys' operands read a phase ahead, the values' behind the first scores,
-// score and value MFMAs taking turns and everything else in the gaps between them: 8192 tokens
-// 539 -> 493 us (1115 TFLOP/s; bf16 GEMMs of this size reach 1350-1600 here), 4096 tokens
-// 146 -> 135, 2000 on 4000 204 -> 165 (same process, graph replays, inputs of unit variance).
+// What bounds it: the two phases and the clock. In steady replays at 8192 tokens the chip runs this
+// kernel at 1.87 GHz (cycle counter over the real-time counter, per work-group; 4096 tokens 1.90;
+// a loop of these MFMAs alone 1.5-1.7, one on 8 CUs 2.4), and a SHARED step takes 0.87 us, of
+// which its MFMAs (8 waves x 16 of 32 cycles, 1024 cycles a SIMD) fill 63 %; softmax phases and
+// barriers, not told apart, keep the matrix cores waiting for the rest. Work-groups are busy 455 of
+// the call's 492 us. The MFMA phase used to wait for its operands: keys read in pairs just
+// before their MFMAs, softmax phases carrying the staging. With the keys' operands read a phase
+// ahead, the values' behind the first scores, score and value MFMAs taking turns and everything
+// else in the gaps between them: 8192 tokens 539 -> 493 us (1115 TFLOP/s; bf16 GEMMs of this size
+// reach 1350-1600 here), 4096 tokens 146 -> 135, 2000 on 4000 204 -> 165 (same process, graph
+// replays, inputs of unit variance).
 //
 // The per-wave MFMA layouts, the exp2-domain online softmax with lazy rescale, the
 // transposing V reads and the output / split-partial formats are those of the
