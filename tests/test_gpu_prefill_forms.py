@@ -186,3 +186,32 @@ def test_prefill_pick(gpu, name):
         ref = orc.attention(q[qsl[b]:qsl[b + 1]], bts[b], seqs[b][0], scale, True, **pools)
         excess = np.abs(ref - got[qsl[b]:qsl[b + 1]]) - (2e-2 + (np.abs(ref) * 2.0 ** -8 if kind == "int8" else 0))
         assert float(np.max(excess)) <= 0, f"sequence {b}: over the tolerance by {np.max(excess)}"
+
+
+@pytest.mark.parametrize("D,seqs,n,start,like", [(128, 1, 600, 0, PAIRED16), (128, 5, 128, 100, PAIRED16),
+                                                 (128, 20, 16, 1008, STAGED), (64, 3, 240, 100, STAGED),
+                                                 (64, 64, 16, 100, STAGED)])
+def test_prefill_form_rounds_no_more(gpu, D, seqs, n, start, like):
+    """The error against 64 bits (2-norm, three seeds) is no larger than that of the kernel that takes
+    such a step otherwise: 0.5 % for the seeds. Without the first steps' eager rescale it was 1.4 to
+    6 % larger, with it 0.3 to 1.6 % smaller."""
+    H, KVH, P = 32, 8, 16
+    per = -(-(start + n) // P)
+    assert pick(n, seqs, P * per, heads=H, kv_heads=KVH, D=D) != NONE
+    norms = np.zeros(2)
+    for seed in range(3):
+        g = rng(5500 + seed + n + D)
+        bts = (g.permutation(seqs * per) + 1).astype(np.int32).reshape(seqs, per)
+        q, kp = randn(g, seqs * n, H, D, bf16=True), randn(g, seqs * per, KVH, P, D, bf16=True)
+        vp = randn(g, seqs * per, KVH, P, D, bf16=True)
+        ref = np.concatenate([orc.attention(q[b * n:(b + 1) * n], bts[b], start, 1 / math.sqrt(D), True, kp, vp)
+                              for b in range(seqs)])
+        qd, k, v = (torch.from_numpy(x).bfloat16().cuda() for x in (q, kp, vp))
+        pos = torch.arange(start, start + n, dtype=torch.int32, device="cuda").repeat(seqs)
+        for i, path in enumerate((ti.TI_PATH_AUTO, like)):
+            out = torch.empty_like(qd)
+            ws = ti.attention_workspace(BE, qd, k, num_seqs=seqs, max_query_len=n, path=path)
+            ti.paged_attention_(BE, out, ws, qd, k, v, torch.from_numpy(bts).cuda(), pos, 1 / math.sqrt(D), max_query_len=n,
+                                path=path)
+            norms[i] += np.linalg.norm(out.float().cpu().numpy() - ref)
+    assert norms[0] <= 1.005 * norms[1], norms[0] / norms[1]

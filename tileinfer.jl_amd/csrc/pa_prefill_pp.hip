@@ -69,6 +69,7 @@ struct PPParams {
     const int32_t *positions, *qsl, *bt;
     float *part;                       // split partials [B][Hk][splits][M][D + 2]
     int bt_stride, num_pages, P, pshift, Hk, Hq, G, TQ, nmax, qtiles, causal, splits, sshift, M;   // splits = 2^sshift
+    int eager;                         // first steps that rescale to every larger maximum
     float scale_log2;
 };
 
@@ -357,8 +358,8 @@ prefill_pp_kernel(PPParams p) {
         }
         sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(ka[i]), qreg[i], sc, 0, 0, 0);
     };
-    // Online softmax of step j's scores (exp2 domain, lazy rescale) -> pb. Only tiles
-    // reaching past mask_from (the diagonal / last tiles) compare key positions.
+    // Online softmax of step j's scores (exp2 domain, lazy rescale after the first p.eager steps)
+    // -> pb. Only tiles reaching past mask_from (the diagonal / last tiles) compare key positions.
     const int jm = min(mask_from + 1, kt_hi * KT); // first key position that a row may not see
     auto softmax = [&](int j) {
         const int kt = tile(j);
@@ -388,7 +389,7 @@ prefill_pp_kernel(PPParams p) {
 #pragma unroll
         for (int e = 0; e < 16; e++) mt = fmaxf(mt, sc[e]);
         if constexpr (!INT8) mt *= p.scale_log2;
-        if (__any(mt > m + RESCALE_LOG2)) {
+        if (__any(mt > m + (j < p.eager ? 0.0f : RESCALE_LOG2))) {
             mt = fmaxf(mt, __shfl_xor(mt, 32));
             const float mn = fmaxf(m, mt);
             const float alpha = fast_exp2(m - mn);
@@ -715,6 +716,17 @@ int ti_launch_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, const
     p.part = (float *)a->workspace;
     p.splits = pl.splits;
     p.sshift = __builtin_ctz(pl.splits);
+    // Every key group's first maximum is a probability of exactly 1, so fewer groups round more on
+    // short contexts. Where the kernels that this one replaces have more groups than the form (four
+    // on 16-row waves and 64-row tiles, eight where they split blocks; two below 1024 work-groups
+    // of 128 rows), its first steps rescale to every larger maximum, which brings the error against
+    // 64 bits to theirs: 600 tokens 0.00196 (KSPLIT without 0.00200, the 16-row kernel 0.00196) for
+    // 16.1 -> 16.5 us, 24 x 16 on 2000 0.00230 (0.00234, 0.00231) for 45.1 -> 45.4, five of 512 at
+    // head_dim 64 0.00198 (SOLO without 0.00204, four-wave 0.00200) for 20.8 -> 21.3.
+    const long long T = (a->max_query_len + 128 / p.G - 1) / (128 / p.G), W = T * p.Hk * a->num_seqs;
+    const bool dense128 = c->kind == TI_KV_DENSE && c->head_dim == 128;
+    if (pl.pp == TI_PP_KSPLIT) p.eager = W > 256 ? 0 : T == 1 ? 8 : 3;
+    else p.eager = W < 1024 && !(T == 1 && dense128) && a->path != TI_PATH_PREFILL_PINGPONG ? 4 : 0;
     p.M = pl.rows;
     p.TQ = pl.TQ;
     p.qtiles = pl.qtiles;
