@@ -132,7 +132,8 @@ PICKS = {
     "block_63": ("bf16", 32, [(40 * (b % 9), 16) for b in range(63)], 0, PAIRED16),
     "block_64": ("bf16", 32, [(40 * (b % 9), 16) for b in range(64)], 0, None),
     "block_int8_32": ("int8", 32, [(40 * (b % 9), 16) for b in range(32)], 2064, PAIRED16),
-    "block_int8_64": ("int8", 32, [(40 * (b % 9), 16) for b in range(64)], 0, PAIRED16),
+    "block_int8_64": ("int8", 32, [(40 * (b % 9), 16) for b in range(64)], 1024, PAIRED16),
+    "block_int8_64_narrow": ("int8", 32, [(40 * (b % 9), 16) for b in range(64)], 0, None),
     "block_int8_65": ("int8", 32, [(40 * (b % 9), 16) for b in range(65)], 0, None),
     # few q-tiles per sequence
     "three_tiles_narrow": ("bf16", 32, [(60, 66)] * 6, 0, PAIRED16),

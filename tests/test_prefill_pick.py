@@ -65,9 +65,18 @@ def test_pick_of_large_launches(want, kw):
     (KSPLIT, dict(n=32, seqs=48, keys=4112, kind=1)),
     (NONE, dict(n=16, seqs=64, keys=4112, kind=1)),
     (SOLO, dict(n=16, seqs=65, keys=4112, kind=1)),
+    (SOLO, dict(n=16, seqs=64, keys=992, kind=1)),
+    (SOLO, dict(n=16, seqs=64, keys=4112, kind=1, D=64)),
+    (NONE, dict(n=16, seqs=63, keys=992, kind=1)),
+    (SOLO, dict(n=92, seqs=24, keys=144, kind=1, total=1476)),
     # INT8: the 16-row kernel's range, tokens held
     (NONE, dict(n=40, seqs=20, keys=2064, kind=1)),
     (NONE, dict(n=119, seqs=5, keys=4112, kind=1, total=357)),
+    (KSPLIT, dict(n=121, seqs=5, keys=144, kind=1)),
+    (NONE, dict(n=121, seqs=5, keys=1008, kind=1)),
+    (NONE, dict(n=121, seqs=5, keys=144, kind=1, total=604)),
+    (NONE, dict(n=128, seqs=8, keys=144, kind=1)),
+    (NONE, dict(n=600, seqs=1, keys=608, kind=1)),
     (NONE, dict(n=1024, seqs=1, keys=4112, kind=1)),
     (KSPLIT, dict(n=1025, seqs=1, keys=4112, kind=1)),
     (KSPLIT, dict(n=1184, seqs=2, keys=4112, kind=1, total=1723)),
@@ -83,7 +92,8 @@ def test_pick_of_large_launches(want, kw):
     (NONE, dict(n=90, seqs=12, keys=144)),
     (KSPLIT, dict(n=90, seqs=12, keys=4112)),
     (NONE, dict(n=256, seqs=8, keys=272, D=64)),
-    (KSPLIT, dict(n=257, seqs=7, keys=272, D=64)),
+    (NONE, dict(n=320, seqs=6, keys=336, D=64)),
+    (KSPLIT, dict(n=321, seqs=5, keys=336, D=64)),
     (KSPLIT, dict(n=256, seqs=8, keys=4112, D=64)),
     (NONE, dict(n=119, seqs=5, keys=4112, total=357, D=64)),
     (KSPLIT, dict(n=119, seqs=5, keys=4112, D=64)),

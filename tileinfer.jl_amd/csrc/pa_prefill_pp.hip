@@ -627,20 +627,23 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     (17 x 16 on 700 19.3 against 29.2), and from W = 192 (24 x 16 on 4096 75.7 against 97.4,
 //     ragged to 4000 61 against 67; to 8000 120 against 115).
 //   One q-tile of up to 64 rows per sequence: none for W < 512, the 16-row kernel's range (32 x
-//     16 on 4096 KSPLIT 98.9 against 91.8, on 200 12.6 against 11.2; INT8 107 against 72, at 64 x
-//     16 SOLO 196 against 150). From there SOLO (96 x 16 on 200 31.0 against 39.8).
-//   INT8 whose 64-row work-groups fit that range: none (20 x 40 on 1000 KSPLIT 64
-//     against 42). Nor for W <= 256, counted by the tokens the sequences hold (5 prompts of 37 to
-//     119 on 800 to 2800 68 against 50): converting tiles doubles the staging there. Beyond, with
-//     few idle rows and more than 40 tiles, KSPLIT (1500 on 4096 206 against 232; two prompts of
-//     520 23.9 against 22.6), but at head_dim 64 only alone (20 x 95 on 3000 142 against 130).
+//     16 on 4096 KSPLIT 98.9 against 91.8, on 200 12.6 against 11.2; INT8 107 against 72, and at
+//     64 x 16 SOLO 196 against 150, but with narrow tables 9.1 against 13.9 for 64 x 9). From there
+//     SOLO (96 x 16 on 200 31.0 against 39.8).
+//   INT8, D = 128, whose 64-row work-groups fit that range: none (20 x 40 on 1000 KSPLIT 64
+//     against 42). Nor does INT8 for W <= 256, counted by the tokens that the sequences hold (5
+//     prompts of 37 to 119 on 800 to 2800 68 against 50): converting tiles doubles the staging there.
+//     But batches of 160 and narrow tables, which leave the contexts little room to differ, take KSPLIT
+//     (5 x 121 from scratch 13.5 against 14.4, D = 64 9.6 against 13.8).
+//     Beyond, with few idle rows and more than 40 tiles, KSPLIT (1500 on 4096 206 against 232; two
+//     prompts of 520 23.9 against 22.6), but at D = 64 only alone (20 x 95 on 3000 142 against 130).
 //   W <= 512: KSPLIT. At most two work-groups per CU, one resident at a time, each with half
 //     the steps of an unsplit q-tile: 520 tokens 15.5 against 16.9 us, 1000 22.5 against 26.2,
 //     2000 46.6 against 55.4; 600 on 4096 65.9 against 114.8; D = 64, 1000 15.6 against 21.8.
 //     q-tiles with rows to spare start later (G = 3: 800 tokens, W = 160, 19.4 against 18.4),
 //     D = 64 by the tokens held (5 chunks of 37 to 119 on 800 to 2800 31.3 against 29.1).
-//     Below 32 tiles and past one round only sequences of more than 8 q-tiles have the steps
-//     (four of 138 to 403 14.5 against 16.3; 12 x 90 19.0, 18.0; D = 64 8 x 256 16.0, 14.9).
+//     Below 32 tiles and past one round only sequences of more than 8 q-tiles (D = 64: 10) have the
+//     steps (four of 138 to 403 14.5 against 16.3; 12 x 90 19.0, 18.0; D = 64 8 x 256 16.0, 14.9).
 //   more: SHARED for dense D = 128 (half the loads and LDS stores per row): 3072 tokens 85.0
 //     against 118.7 us, 8192 493 against 539; else SOLO, whose work-groups share a CU (two,
 //     D = 64 three) and hide each other's fixed cost: INT8 3072 tokens 110.8 against 145.8,
@@ -652,8 +655,8 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     512 on 4096 609, 534).
 // Over 3757 shapes on either side of these lines, of up to 128 sequences, uniform and ragged, steps
 // take 0.87 times as long in the mean as on the kernels that took them before this one had forms.
-// Slower by more than 3 %: 15, nearly all batches of W < 200 whose contexts are ragged, which the
-// host cannot see (7 x 66 on 200 to 930 21.8 against 18.4; 5 x 110 on 1000 each 23.6 against 36.0).
+// Slower by more than 3 %: 14, mostly batches of W < 200 whose contexts are ragged, which the host
+// cannot see (7 x 66 on 200 to 930 21.6 against 18.5; 5 x 110 on 1000 each 23.6 against 36.0).
 int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path, bool bound_keys) {
     const int G = a->q_heads / c->kv_heads, P = c->page_size, D = c->head_dim;
     if (a->dtype != TI_BF16 || (D != 64 && D != 128) || P < 16 || (P & (P - 1)) || G > 64 ||
@@ -672,14 +675,16 @@ int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int pat
     // (unbounded tiles) that answers KSPLIT is right for narrower tables too.
     if (q64 < 256)
         return dense && (dense128 || T > 2) && tiles >= 32 && W >= (tiles <= 40 ? 129 : 192) ? TI_PP_KSPLIT : TI_PP_NONE;
-    if (T == 1 && q64 == W && W < (dense ? 512 : 513)) return TI_PP_NONE;
-    if (!dense && W > 256 && q64 <= 512) return TI_PP_NONE;
+    const bool int8_128 = !dense && D == 128;
+    if (T == 1 && q64 == W && W < (int8_128 && tiles >= 32 ? 513 : 512)) return TI_PP_NONE;
+    if (int8_128 && W > 256 && W < 512 && q64 <= 512) return TI_PP_NONE;
     if (T <= 2 && W >= 512) return TI_PP_SOLO;
-    if (tiles < 32 && W > 256 && W <= 512 && (T > 1 || !dense) && T <= 8) return TI_PP_NONE;
+    if (tiles < 32 && W > 256 && W <= 512 && (T > 1 || !dense) && T <= (D == 64 ? 10 : 8)) return TI_PP_NONE;
     if (T <= 2) return D == 128 && W >= (dense ? 129 : 256) ? TI_PP_KSPLIT : TI_PP_NONE;
     const long long held = W * a->total_tokens / (n * a->num_seqs);
     if (!dense) {
-        if (W <= 640) W = held;
+        if (a->num_seqs > 1 && tiles < 32 && W < 256 && held >= 160) return TI_PP_KSPLIT;
+        if (W <= 512 || (W <= 640 && tiles > 40)) W = held;
         if (W < (D == 64 && a->num_seqs == 1 ? 256 : 257)) return TI_PP_NONE;
         if (W > 512) return TI_PP_SOLO;
         return tiles > 40 && (D == 128 || a->num_seqs == 1) ? TI_PP_KSPLIT : TI_PP_NONE;
