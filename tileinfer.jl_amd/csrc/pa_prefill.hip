@@ -1278,9 +1278,10 @@ ti_prefill_plan ti_plan_prefill(const ti_attention_args *a, const ti_kv_cache *c
     // plan's four-wave kernel (same process) 11.4 -> 10.4 us at 512 tokens, 22.0 -> 19.7 us
     // for 512 on a 1024-token prefix, 27.2 -> 24.6 us at 1024 tokens, 46.3 -> 42.9 us for
     // 1024 on 1024, even at 768 tokens (384 work-groups), but 37.0 -> 43.3 us at 1536 tokens
-    // (768) and twice as slow from 2048 tokens. On a dense cache the ping-pong kernel takes
-    // launches of more than 256 pairs first. The 32-row paired kernel (pinned with
-    // TI_PATH_PREFILL_PAIRED) needs the plan's two-wave, four-group shape.
+    // (768) and twice as slow from 2048 tokens. Most launches of more
+    // than 128 work-groups of 128 rows have gone to a ping-pong form before this
+    // (ti_pick_prefill_pp). The 32-row paired kernel (pinned with TI_PATH_PREFILL_PAIRED)
+    // needs the plan's two-wave, four-group shape.
     // (INT8 caches pair on the 16-row kernel only, its tiles staged through registers)
     const bool i8_ok = c->kind == TI_KV_INT8 && a->dtype == TI_BF16 && c->head_dim == 128 &&
                        c->page_size >= 16 && (c->page_size & (c->page_size - 1)) == 0;

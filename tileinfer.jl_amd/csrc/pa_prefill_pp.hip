@@ -624,8 +624,8 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //   q64 < 256: none. From 32 tiles the four-wave plan's key splits even out ragged contexts (17 x
 //     16 tokens on 500 to 4000: 46 us, KSPLIT 57); below, unsplit, it is the 16-row kernel (17 x
 //     16 on 200 9.9, KSPLIT 11.3; 6 x 66 from scratch 7.8, 9.8). But KSPLIT from 32 to 40 tiles
-//     (17 x 16 on 700 19.3 against 29.2), and from W = 192 (24 x 16 on 4096 75.7 against 97.4,
-//     ragged to 4000 61 against 67; to 8000 120 against 115).
+//     (17 x 16 on 700 20.0 against 29.4), and from W = 192 (24 x 16 on 4096 80.5 against 99.3,
+//     ragged to 4000 65 against 70; to 8000 120 against 115).
 //   One q-tile of up to 64 rows per sequence: none for W < 512, the 16-row kernel's range (32 x
 //     16 on 4096 KSPLIT 98.9 against 91.8, on 200 12.6 against 11.2; INT8 107 against 72, and at
 //     64 x 16 SOLO 196 against 150, but with narrow tables 9.1 against 13.9 for 64 x 9). From there
@@ -634,19 +634,19 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     against 42). Nor does INT8 for W <= 256, counted by the tokens that the sequences hold (5
 //     prompts of 37 to 119 on 800 to 2800 68 against 50): converting tiles doubles the staging there.
 //     But batches of 160 and narrow tables, which leave the contexts little room to differ, take KSPLIT
-//     (5 x 121 from scratch 13.5 against 14.4, D = 64 9.6 against 13.8).
+//     (5 x 121 from scratch 13.7 against 14.5, D = 64 9.7 against 13.8).
 //     Beyond, with few idle rows and more than 40 tiles, KSPLIT (1500 on 4096 206 against 232; two
 //     prompts of 520 23.9 against 22.6), but at D = 64 only alone (20 x 95 on 3000 142 against 130).
 //   W <= 512: KSPLIT. At most two work-groups per CU, one resident at a time, each with half
-//     the steps of an unsplit q-tile: 520 tokens 15.5 against 16.9 us, 1000 22.5 against 26.2,
-//     2000 46.6 against 55.4; 600 on 4096 65.9 against 114.8; D = 64, 1000 15.6 against 21.8.
+//     the steps of an unsplit q-tile: 520 tokens 15.5 against 16.8 us, 1000 22.9 against 26.4,
+//     2000 46.2 against 56.2; 600 on 4096 64.5 against 114.5; D = 64, 1000 16.0 against 21.5.
 //     q-tiles with rows to spare start later (G = 3: 800 tokens, W = 160, 19.4 against 18.4),
 //     D = 64 by the tokens held (5 chunks of 37 to 119 on 800 to 2800 31.3 against 29.1).
 //     Below 32 tiles and past one round only sequences of more than 8 q-tiles (D = 64: 10) have the
 //     steps (four of 138 to 403 14.5 against 16.3; 12 x 90 19.0, 18.0; D = 64 8 x 256 16.0, 14.9).
-//   more: SHARED for dense D = 128 (half the loads and LDS stores per row): 3072 tokens 85.0
-//     against 118.7 us, 8192 493 against 539; else SOLO, whose work-groups share a CU (two,
-//     D = 64 three) and hide each other's fixed cost: INT8 3072 tokens 110.8 against 145.8,
+//   more: SHARED for dense D = 128 (half the loads and LDS stores per row): 3072 tokens 88.7
+//     against 119.4 us, 8192 493 against 539; else SOLO, whose work-groups share a CU (two,
+//     D = 64 three) and hide each other's fixed cost: INT8 3072 tokens 116.4 against 147.4,
 //     D = 64 8192 309 against 394, eight D = 64 prompts of 100 to 2000 tokens 58.8 against
 //     78.3. SOLO also takes dense D = 128 batches whose sequences are short in queries and keys (16
 //     x 300 tokens 39.8 against 42.1 on SHARED, 16 x 512 71.9, 74.9) or mostly absent (a prompt of
@@ -655,7 +655,7 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     512 on 4096 609, 534).
 // Over 3757 shapes on either side of these lines, of up to 128 sequences, uniform and ragged, steps
 // take 0.87 times as long in the mean as on the kernels that took them before this one had forms.
-// Slower by more than 3 %: 14, mostly batches of W < 200 whose contexts are ragged, which the host
+// Slower by more than 3 %: 16, mostly batches of W < 200 whose contexts are ragged, which the host
 // cannot see (7 x 66 on 200 to 930 21.6 against 18.5; 5 x 110 on 1000 each 23.6 against 36.0).
 int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path, bool bound_keys) {
     const int G = a->q_heads / c->kv_heads, P = c->page_size, D = c->head_dim;
@@ -726,8 +726,9 @@ int ti_launch_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, const
     // on 16-row waves and 64-row tiles, eight where they split blocks; two below 1024 work-groups
     // of 128 rows), its first steps rescale to every larger maximum, which brings the error against
     // 64 bits to theirs: 600 tokens 0.00196 (KSPLIT without 0.00200, the 16-row kernel 0.00196) for
-    // 16.1 -> 16.5 us, 24 x 16 on 2000 0.00230 (0.00234, 0.00231) for 45.1 -> 45.4, five of 512 at
-    // head_dim 64 0.00198 (SOLO without 0.00204, four-wave 0.00200) for 20.8 -> 21.3.
+    // 16.1 -> 16.5 us, 24 x 16 on 2000 0.00230 (0.00234, 0.00231) for 45.1 -> 45.4 (on 4096 77.0 ->
+    // 80.5), five of 512 at head_dim 64 0.00198 (SOLO without 0.00204, four-wave 0.00200) for 20.8
+    // -> 21.3.
     const long long T = (a->max_query_len + 128 / p.G - 1) / (128 / p.G), W = T * p.Hk * a->num_seqs;
     const bool dense128 = c->kind == TI_KV_DENSE && c->head_dim == 128;
     if (pl.pp == TI_PP_KSPLIT) p.eager = W > 256 ? 0 : T == 1 ? 8 : 3;
