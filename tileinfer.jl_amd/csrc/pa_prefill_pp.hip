@@ -655,7 +655,7 @@ void launch_pp_form(const PPParams &p, int form, int B, hipStream_t s) {
 //     512 on 4096 609, 534).
 // Over 3757 shapes on either side of these lines, of up to 128 sequences, uniform and ragged, steps
 // take 0.87 times as long in the mean as on the kernels that took them before this one had forms.
-// Slower by more than 3 %: 16, mostly batches of W < 200 whose contexts are ragged, which the host
+// Slower by more than 3 %: 14, mostly batches of W < 200 whose contexts are ragged, which the host
 // cannot see (7 x 66 on 200 to 930 21.6 against 18.5; 5 x 110 on 1000 each 23.6 against 36.0).
 int ti_pick_prefill_pp(const ti_attention_args *a, const ti_kv_cache *c, int path, bool bound_keys) {
     const int G = a->q_heads / c->kv_heads, P = c->page_size, D = c->head_dim;
